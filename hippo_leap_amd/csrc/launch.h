@@ -163,13 +163,14 @@ hipError_t prefill_mfma_launch(const PrefillLaunch& p, hipStream_t stream);
 int prefill_mfma_tpad(int seq_len);
 
 // ---- fp32 linear layer (linear.hip) ----------------------------------------
-// Y[M, T] = W[M, K] . X[K, T]: GEMV for T == 1, fp32-MFMA GEMM otherwise.
+// Y[M, T] = W[M, K] . X[K, T]: GEMV for T == 1, GEMM on split operands otherwise.
 struct LinearPlan {
   bool gemv;
-  bool vec;      // 16-byte loads (K % 4 == 0, T % 4 == 0 for the GEMM, aligned w, x)
+  bool vec;      // GEMV: 16-byte loads (K % 4 == 0, aligned w, x)
   int wpr;       // GEMV: waves per row (1, or 4 when M is small)
-  int tile;      // GEMM: output tile edge (64 or 128)
-  int grid_x, grid_y;
+  int grid_x;    // GEMV
+  int variant;   // GEMM: index into the split GEMM's variants
+  int tiles_m, tiles_n;
 };
 LinearPlan linear_plan(int M, int K, int T, const float* w, const float* x);
 hipError_t linear_col_launch(float* y, const float* x, const float* w, int K, int M, int T,

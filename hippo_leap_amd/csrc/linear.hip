@@ -14,24 +14,21 @@
 //   small, so the grid still covers the chip), one cross-lane reduction per
 //   row.  x is re-read from L2 by every wave (staging it in LDS measured
 //   slower).
-// * T > 1 (prefill): linear_mfma_kernel on fp32 MFMA
-//   (v_mfma_f32_32x32x2_f32); the bound is the fp32 matrix peak over
-//   2*M*K*T FLOPs.  Workgroup tiles of 128x128 outputs (4 waves, 2x2 blocks
-//   of 32x32 each) when there are enough of them to fill the chip, else
-//   64x64 (8 waves in two K halves); K staged through double-buffered LDS
-//   with two chunks in flight in registers, one barrier per chunk.
+// * T > 1 (prefill): linear_split_kernel, three fp16 MFMAs
+//   (v_mfma_f32_32x32x16_f16) on hi/lo parts of the fp32 operands per fp32
+//   product; fp32 MFMAs for the output tiles where that is not possible.
 //
 // Accumulation is fp32 as in the reference; only the summation order
 // differs (the reference's decode kernel reduces 256 strided partial sums,
 // its prefill kernel sums k = 0..K-1 in order).
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 #include "launch.h"
 
 namespace hl {
 namespace {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 __device__ inline float wave_sum(float v) {
 #pragma unroll
@@ -109,184 +106,436 @@ __global__ __launch_bounds__(256) void linear_gemv_kernel(const float* __restric
 }
 
 // ---------------------------------------------------------------------------
-// GEMM (T > 1) on fp32 MFMA
+// GEMM (T > 1) on fp16 MFMA over split fp32 operands
 // ---------------------------------------------------------------------------
-// v_mfma_f32_32x32x2_f32: lane l supplies A[m = l%32][k = l/32] and
-// B[k = l/32][n = l%32]; output element e of lane l is C[8(e/4) + 4(l/32) +
-// e%4][l%32].  Within each group of 8 k, MFMA step i pairs k = 8g + i (lane
-// half 0) with k = 8g + 4 + i (half 1), so a lane's four A values for the
-// group are one contiguous 16-byte LDS read.
+// Every operand x becomes x s = hi + lo, hi = f16(x s), lo = f16(x s - hi),
+// s a power of two per row of W and per column of X; a product is then
+// hi hi' + hi lo' + lo hi' into one fp32 accumulator (lo lo' is below 2^-22
+// of it).  That costs 3 x 32 matrix-core cycles per 32x32x16 block where
+// v_mfma_f32_32x32x2_f32 takes 8 x 64.  Error: 2^-23 of each element and
+// 2^-25 absolute after scaling (the MFMA takes f16 subnormals as they are),
+// below the fp32 accumulation's own: against a 64-bit product
+// 2.6e-7 at K = 4096 and 2.0e-7 at 2048 where fp32 MFMAs gave 1.1e-6 and
+// 4.1e-7 (one accumulation chain of K instead of KW chains of 16-long sums).
 //
-// The 2x2 waves of a workgroup each own a (32*WM) x (32*WN) block of the
-// (64*WM) x (64*WN) output tile.  KW = 2 doubles the workgroup to 8 waves:
-// waves 4..7 take the upper half of every K chunk for the same blocks (two
-// waves per SIMD to cover each other's LDS and barrier waits), and their
-// sums are added through LDS at the end.
-template <int WM, int WN, int BK, int KW, bool VEC, int PF = 2>
-__global__ __launch_bounds__(256 * KW) void linear_mfma_kernel(const float* __restrict__ w,
-                                                          const float* __restrict__ x,
-                                                          float* __restrict__ y, int M, int K,
-                                                          int T) {
-  constexpr int BM = 64 * WM, BN = 64 * WN;
-  // Row pitches in floats.  SA = 36: the 16 lanes served together by one
-  // ds_read_b128 (rows m..m+15, same k) start on distinct 4-bank groups.
-  // SB = BN + 8: rows k and k + 4 (the two lane halves of a b32 read) sit
-  // 32 banks apart, so the 64 lanes hit 64 distinct banks.
-  constexpr int SA = BK + 4, SB = BN + 8;
-  constexpr int NTH = 256 * KW;
-  constexpr int NA = BM * BK / 4 / NTH;  // 16-byte A chunks per thread
-  constexpr int NB = BK * BN / 4 / NTH;  // 16-byte B chunks per thread
-  static_assert(NA * NTH * 4 == BM * BK && NB * NTH * 4 == BK * BN, "tile / thread mismatch");
-  __shared__ __attribute__((aligned(16))) float sA[2][BM * SA];
-  __shared__ __attribute__((aligned(16))) float sB[2][BK * SB];
+// s brings the largest magnitude of the first 16 k that a wave meets into
+// [64, 128): the absolute error is then 2^-31 of it, and later elements may
+// be 2^9 times larger.  One above that, an inf or a NaN makes a partial sum inf or NaN, and the workgroup then computes its
+// tile once more with fp32 MFMAs (body<false>), so that inf and NaN come out
+// as fp32 arithmetic gives them.  A row or column whose first 16 elements are
+// zero is scanned for its largest element instead.
+//
+// The KW waves of a workgroup share one (32 WM) x (32 WN) output tile and
+// split K between them in chunks of CK (wave w takes chunks w, w + KW, ...),
+// each with its own staging area: no barrier until the partial sums meet in
+// LDS.  W comes in rows of 4 CK bytes through LDS (16-byte pieces swizzled by
+// the row, fp32; every wave splits what it reads itself); X goes straight to
+// registers, XD 16-k steps ahead: lane ln of a half holds columns
+// WN ln .. WN ln + WN - 1 of 8 k, so one load of 4 WN bytes serves the WN
+// column blocks, and neither K nor T nor an address has to be a multiple of
+// anything.  The splits cost 2 (multiply) + 2 (v_cvt_pk_f16_f32) + 4
+// (v_fma_mix_f32) + 2 cycles per element and lane; v_fma_mixlo_f16, which
+// would take two instructions, measured 8 cycles each.
+//
+// What bounds it: bytes into the CUs on the small tiles (128 B per k of a
+// 64x64 tile from L2; the prefetch depth did not matter), the matrix cores
+// at three products on 64x128 tiles.  Before: fp32 MFMAs on 128x128 tiles
+// staged through LDS, scalar loads whenever K or T was no multiple of 4.
+//   M x K, T              before      now
+//   4096 x 4096,    37    130 us     20.7   (32x32 tiles)
+//   2048 x 2048,   301     76        23     (64x64)
+//   2048 x 8192,   301    267        70     (64x64)
+//   14336 x 4096, 1000   1080       479     (64x128: 245 TFLOP/s)
+//   4096 x 4096,  4096   1044       521     (64x128: 264 TFLOP/s)
+// Measured and not kept: x loads four steps ahead (no change), 64-k chunks on
+// 64x64 tiles (17% slower), sixteen waves (slower), 128x64 and 128x128 tiles.
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = tid >> 6;
-  const int ln = lane & 31, hh = lane >> 5;
-  const int kg = wave >> 2;  // K half of each chunk (KW = 2)
-  const int wm = (wave >> 1) & 1, wn = wave & 1;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-
-  f32x4 ra[PF][NA], rb[PF][NB];  // PF chunks in flight, one register set each
-  auto load = [&](int c, int st) {
-    const int k0 = c * BK;
+// N floats at a 4-byte aligned address.
+template <int N>
+struct FVec {
+  typedef float T __attribute__((ext_vector_type(N), aligned(4)));
+};
+template <int N>
+__device__ __forceinline__ void load_n(const float* p, float* v) {
+  if constexpr (N == 1) {
+    v[0] = *p;
+  } else {
+    const typename FVec<N>::T t = *(const typename FVec<N>::T*)p;
 #pragma unroll
-    for (int j = 0; j < NA; ++j) {
-      const int idx = tid + NTH * j, r = idx / (BK / 4), kk = k0 + 4 * (idx % (BK / 4));
-      const int m = m0 + r;
-      if (VEC) {
-        ra[st][j] = (m < M && kk < K) ? *(const f32x4*)(w + (size_t)m * K + kk) : f32x4{0.f, 0.f, 0.f, 0.f};
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          ra[st][j][e] = (m < M && kk + e < K) ? w[(size_t)m * K + kk + e] : 0.f;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int idx = tid + NTH * j, r = idx / (BN / 4), n = n0 + 4 * (idx % (BN / 4));
-      const int k = k0 + r;
-      if (VEC) {
-        rb[st][j] = (k < K && n < T) ? *(const f32x4*)(x + (size_t)k * T + n) : f32x4{0.f, 0.f, 0.f, 0.f};
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          rb[st][j][e] = (k < K && n + e < T) ? x[(size_t)k * T + n + e] : 0.f;
-      }
-    }
-  };
-  auto store = [&](int buf, int st) {
-#pragma unroll
-    for (int j = 0; j < NA; ++j) {
-      const int idx = tid + NTH * j;
-      *(f32x4*)&sA[buf][(idx / (BK / 4)) * SA + 4 * (idx % (BK / 4))] = ra[st][j];
-    }
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int idx = tid + NTH * j;
-      *(f32x4*)&sB[buf][(idx / (BN / 4)) * SB + 4 * (idx % (BN / 4))] = rb[st][j];
-    }
-  };
-
-  // Independent accumulation chains per output block: back-to-back MFMAs
-  // into one accumulator wait for each other, so with a single 32x32 block
-  // per wave the k-steps rotate over CH accumulators (summed at the end).
-  constexpr int CH = (WM * WN >= 2) ? 1 : 2;
-  f32x16 acc[WM][WN][CH];
-#pragma unroll
-  for (int a = 0; a < WM; ++a)
-#pragma unroll
-    for (int b = 0; b < WN; ++b)
-#pragma unroll
-      for (int h = 0; h < CH; ++h)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[a][b][h][e] = 0.f;
-
-  auto compute = [&](int buf) {
-    const float* pa = &sA[buf][(wm * 32 * WM + ln) * SA + 4 * hh];
-    const float* pb = &sB[buf][(4 * hh) * SB + wn * 32 * WN + ln];
-    constexpr int GPW = BK / 8 / KW;  // groups of 8 k per wave and chunk
-#pragma unroll
-    for (int g = kg * GPW; g < (kg + 1) * GPW; ++g) {
-      f32x4 af[WM];
-      float bf[WN][4];
-#pragma unroll
-      for (int a = 0; a < WM; ++a) af[a] = *(const f32x4*)(pa + a * 32 * SA + 8 * g);
-#pragma unroll
-      for (int b = 0; b < WN; ++b)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) bf[b][i] = pb[(8 * g + i) * SB + b * 32];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int a = 0; a < WM; ++a)
-#pragma unroll
-          for (int b = 0; b < WN; ++b)
-            acc[a][b][i % CH] =
-                __builtin_amdgcn_mfma_f32_32x32x2f32(af[a][i], bf[b][i], acc[a][b][i % CH], 0, 0, 0);
-    }
-  };
-
-  // Chunk j travels in register set j % PF: chunks 0..PF-1 are requested up
-  // front, and each iteration refills the set it has just written to LDS
-  // with the chunk PF further on.
-  const int nk = (K + BK - 1) / BK;
-#pragma unroll
-  for (int st = 0; st < PF; ++st)
-    if (st < nk) load(st, st);
-  store(0, 0);
-  if (PF < nk) load(PF, 0);
-  __syncthreads();
-  for (int c0 = 0; c0 < nk; c0 += PF) {
-#pragma unroll
-    for (int q = 0; q < PF; ++q) {
-      const int c = c0 + q;
-      if (c < nk) {
-        compute(c & 1);
-        const int st = (q + 1) % PF;
-        if (c + 1 < nk) store((c + 1) & 1, st);
-        if (c + 1 + PF < nk) load(c + 1 + PF, st);
-        __syncthreads();
-      }
-    }
+    for (int i = 0; i < N; ++i) v[i] = t[i];
   }
+}
 
-  float* red = sA[0];  // KW = 2: the upper waves' sums, [wave][a][b][e][lane]
-  if (KW == 2 && kg == 1) {
+// x s - hi in fp32, hi the low (J = 0) or high half of a packed f16 pair.
+template <int J>
+__device__ __forceinline__ float split_rest(float x, float s, uint32_t hi) {
+  float r;
+  if constexpr (J == 0) asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(r) : "v"(x), "v"(s), "v"(hi));
+  else asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r) : "v"(x), "v"(s), "v"(hi));
+  return r;
+}
+__device__ __forceinline__ uint32_t pack_f16(float a, float b) {
+  return __builtin_bit_cast(uint32_t, f16x2{(_Float16)a, (_Float16)b});
+}
+__device__ __forceinline__ void split8(const float* v, float s, f16x8& hi, f16x8& lo) {
+  u32x4 h, l;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) h[j] = pack_f16(v[2 * j] * s, v[2 * j + 1] * s);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    l[j] = pack_f16(split_rest<0>(v[2 * j], s, h[j]), split_rest<1>(v[2 * j + 1], s, h[j]));
+  hi = __builtin_bit_cast(f16x8, h);
+  lo = __builtin_bit_cast(f16x8, l);
+}
+
+// The power of two that brings magnitude m into [64, 128) (1 for m = 0).  bad:
+// m is outside 2^-100 .. 2^100, inf or NaN.
+__device__ __forceinline__ float split_scale(float m, bool& bad) {
+  const uint32_t e = __float_as_uint(m) >> 23;
+  if (m == 0.f) return 1.f;
+  bad = bad || e < 27u || e > 227u;
+  return __uint_as_float((260u - e) << 23);
+}
+
+// Orders a wave's LDS writes and reads (each wave has its own staging area).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// group_m: tiles are walked group_m row tiles at a time, row tiles fastest.
+template <int WM, int WN, int KW, int CK, int XD>
+__global__ __launch_bounds__(64 * KW) void linear_split_kernel(const float* __restrict__ w,
+                                                               const float* __restrict__ x,
+                                                               float* __restrict__ y, int M, int K, int T,
+                                                               int tiles_m, int tiles_n, int group_m) {
+  constexpr int ST = CK / 16;            // 16-k steps per chunk
+  constexpr int BM = 32 * WM, BN = 32 * WN;
+  constexpr int C16 = CK / 4;            // 16-byte pieces per staged row
+  constexpr int NL = BM * CK / 4 / 64;   // 16-byte loads per lane and chunk
+  constexpr int RPL = 64 / C16;          // rows per load
+  constexpr int STAGE = BM * CK;         // floats of a wave's staging area
+  constexpr int PART = BM * BN;          // floats of a wave's partial sums
+  static_assert(XD <= ST && ST % XD == 0, "x buffers");
+  __shared__ __attribute__((aligned(16))) float lds[KW * (STAGE > PART ? STAGE : PART)];
+  __shared__ __attribute__((aligned(16))) float inv_row[KW][BM];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ln = lane & 31, hh = lane >> 5;
+
+  // Each XCD (workgroup id mod 8) walks its own contiguous run of tiles, so
+  // that its L2 serves the rows and columns its workgroups share.
+  const int total = tiles_m * tiles_n, xcd = blockIdx.x % 8, rem = total % 8;
+  const int id = xcd * (total / 8) + min(xcd, rem) + (int)blockIdx.x / 8;
+  const int gi = id / (group_m * tiles_n), in = id - gi * (group_m * tiles_n);
+  const int gm = min(group_m, tiles_m - gi * group_m);
+  const int m0 = (gi * group_m + in % gm) * BM, n0 = (in / gm) * BN;
+
+  float* stage = lds + wave * STAGE;
+  const int lrow = lane / C16, lp = lane % C16;
+  // This lane's first column; the last lanes move back so that their WN
+  // columns stay inside the row (and store only their own).
+  const int nom = n0 + WN * ln, col0 = min(nom, T - WN);
+  const float* wt = w + (size_t)m0 * K;
+  const int mlast = M - 1 - m0;  // rows past it read row mlast and store nothing
+  uint32_t woff[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const int r = RPL * i + lrow;
+    woff[i] = (uint32_t)min(r, mlast) * (uint32_t)K + 4u * (uint32_t)(lp ^ (r & (C16 - 1)));
+  }
+  const uint32_t xoff = (uint32_t)(8 * hh) * (uint32_t)T + (uint32_t)col0;
+  const int nfull = K / CK;
+  const int nmine = wave < nfull ? (nfull - wave + KW - 1) / KW : 0;  // full chunks of this wave
+  const bool tail = K % CK != 0 && wave == nfull % KW;                 // the last, partial chunk
+
+  f32x16 acc[WM][WN];
+
+  // This wave's share of K into acc, on split operands or (false) on fp32
+  // MFMAs.  Returns true when the split operands cannot hold a value.
+  auto body = [&](auto split_tag) -> bool {
+    constexpr bool SPLIT = decltype(split_tag)::value;
 #pragma unroll
     for (int a = 0; a < WM; ++a)
 #pragma unroll
       for (int b = 0; b < WN; ++b)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          float v = acc[a][b][0][e];
+        for (int e = 0; e < 16; ++e) acc[a][b][e] = 0.f;
+    f32x4 wr[NL];
+    float xr[XD][8][WN];
+    [[maybe_unused]] float sa[WM], sb[WN];
+    auto load_w = [&](int c) {
+      const float* src = wt + (size_t)c * CK;
 #pragma unroll
-          for (int h = 1; h < CH; ++h) v += acc[a][b][h][e];
-          red[((((wave & 3) * WM + a) * WN + b) * 16 + e) * 64 + lane] = v;
+      for (int i = 0; i < NL; ++i) {
+        const FVec<4>::T t = *(const FVec<4>::T*)(src + woff[i]);
+        wr[i] = f32x4{t[0], t[1], t[2], t[3]};
+      }
+    };
+    auto load_x = [&](int k0, float (*xv)[WN]) {
+      const float* src = x + (size_t)k0 * T;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) load_n<WN>(src + (size_t)j * T + xoff, xv[j]);
+    };
+    auto put_w = [&]() {
+#pragma unroll
+      for (int i = 0; i < NL; ++i) *(f32x4*)(stage + (RPL * i + lrow) * CK + 4 * lp) = wr[i];
+      wave_lds_sync();
+    };
+    // k 16 s + 8 hh .. + 7 of staged row 32 a + ln
+    auto read_a = [&](int a, int s, float* v) {
+      const int r = 32 * a + ln, sw = r & (C16 - 1);
+      const f32x4 v0 = *(const f32x4*)(stage + r * CK + 4 * ((4 * s + 2 * hh) ^ sw));
+      const f32x4 v1 = *(const f32x4*)(stage + r * CK + 4 * ((4 * s + 2 * hh + 1) ^ sw));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = v0[j], v[4 + j] = v1[j];
+    };
+    auto scales = [&](const float (*xv)[WN]) -> bool {
+      float ma[WM], mb[WN];
+      bool zero = false, bad = false;
+#pragma unroll
+      for (int a = 0; a < WM; ++a) {
+        float v[8];
+        read_a(a, 0, v);
+        ma[a] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ma[a] = fmaxf(ma[a], fabsf(v[j]));
+        ma[a] = fmaxf(ma[a], __shfl_xor(ma[a], 32, 64));
+        zero = zero || ma[a] == 0.f;
+      }
+#pragma unroll
+      for (int b = 0; b < WN; ++b) {
+        mb[b] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mb[b] = fmaxf(mb[b], fabsf(xv[j][b]));
+        mb[b] = fmaxf(mb[b], __shfl_xor(mb[b], 32, 64));
+        zero = zero || mb[b] == 0.f;
+      }
+      if (__any(zero)) {  // rare: the largest elements of this wave's whole share
+        for (int c = wave; c * CK < K; c += KW)
+          for (int k = c * CK + hh; k < min(c * CK + CK, K); k += 2) {
+#pragma unroll
+            for (int a = 0; a < WM; ++a)
+              ma[a] = fmaxf(ma[a], fabsf(wt[(size_t)min(32 * a + ln, mlast) * K + k]));
+#pragma unroll
+            for (int b = 0; b < WN; ++b) mb[b] = fmaxf(mb[b], fabsf(x[(size_t)k * T + col0 + b]));
+          }
+#pragma unroll
+        for (int a = 0; a < WM; ++a) ma[a] = fmaxf(ma[a], __shfl_xor(ma[a], 32, 64));
+#pragma unroll
+        for (int b = 0; b < WN; ++b) mb[b] = fmaxf(mb[b], __shfl_xor(mb[b], 32, 64));
+      }
+#pragma unroll
+      for (int a = 0; a < WM; ++a) {
+        sa[a] = split_scale(ma[a], bad);
+        if (hh == 0) inv_row[wave][32 * a + ln] = 1.0f / sa[a];
+      }
+#pragma unroll
+      for (int b = 0; b < WN; ++b) sb[b] = split_scale(mb[b], bad);
+      wave_lds_sync();
+      return __any(bad);
+    };
+    auto step = [&](int s, const float (*xv)[WN]) {
+      if constexpr (SPLIT) {
+        f16x8 ah[WM], al[WM];
+#pragma unroll
+        for (int a = 0; a < WM; ++a) {
+          float v[8];
+          read_a(a, s, v);
+          split8(v, sa[a], ah[a], al[a]);
         }
-  }
-  if (KW == 2) __syncthreads();
-  if (kg == 1) return;
 #pragma unroll
-  for (int a = 0; a < WM; ++a)
+        for (int b = 0; b < WN; ++b) {
+          float v[8];
 #pragma unroll
-    for (int b = 0; b < WN; ++b) {
-      const int n = n0 + wn * 32 * WN + b * 32 + ln;
+          for (int j = 0; j < 8; ++j) v[j] = xv[j][b];
+          f16x8 bh, bl;
+          split8(v, sb[b], bh, bl);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int m = m0 + wm * 32 * WM + a * 32 + 8 * (e >> 2) + 4 * hh + (e & 3);
-        float v = acc[a][b][0][e];
+          for (int a = 0; a < WM; ++a)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[a], bh, acc[a][b], 0, 0, 0);
 #pragma unroll
-        for (int h = 1; h < CH; ++h) v += acc[a][b][h][e];
-        if (KW == 2) v += red[(((wave * WM + a) * WN + b) * 16 + e) * 64 + lane];
-        if (m < M && n < T) y[(size_t)m * T + n] = v;
+          for (int a = 0; a < WM; ++a)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[a], bl, acc[a][b], 0, 0, 0);
+#pragma unroll
+          for (int a = 0; a < WM; ++a)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[a], bh, acc[a][b], 0, 0, 0);
+        }
+      } else {
+        // MFMA j pairs k 8 hh + j of the two lane halves
+#pragma unroll
+        for (int a = 0; a < WM; ++a) {
+          float v[8];
+          read_a(a, s, v);
+#pragma unroll
+          for (int b = 0; b < WN; ++b)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[j], xv[j][b], acc[a][b], 0, 0, 0);
+        }
+      }
+    };
+    bool scaled = false;
+    if (nmine > 0) {
+      // The loads are unconditional (the last ones repeat the last chunk and
+      // are not used) and kept in program order, so that every wait counts
+      // the loads behind it exactly.
+      load_w(wave);
+#pragma unroll
+      for (int s = 0; s < XD; ++s) load_x(wave * CK + 16 * s, xr[s]);
+      for (int n = 0, c = wave; n < nmine; ++n, c += KW) {
+        put_w();
+        const int cn = min(c + KW, nfull - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(cn);
+        __builtin_amdgcn_sched_barrier(0);
+        if (SPLIT && n == 0) {
+          if (scales(xr[0])) return true;
+          scaled = true;
+        }
+#pragma unroll
+        for (int s = 0; s < ST; ++s) {
+          step(s, xr[s % XD]);
+          __builtin_amdgcn_sched_barrier(0);
+          load_x(s + XD < ST ? c * CK + 16 * (s + XD) : cn * CK + 16 * (s + XD - ST), xr[s % XD]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     }
+    if (tail) {
+      const int k0 = nfull * CK;
+#pragma unroll
+      for (int i = 0; i < NL; ++i) {
+        const int r = RPL * i + lrow, kk = k0 + 4 * (lp ^ (r & (C16 - 1)));
+        const float* src = wt + (size_t)min(r, mlast) * K;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = src[min(kk + e, K - 1)];
+          wr[i][e] = kk + e < K ? v : 0.f;
+        }
+      }
+      wave_lds_sync();
+      put_w();
+      for (int s = 0; s < ST && k0 + 16 * s < K; ++s) {
+        const int kb = k0 + 16 * s + 8 * hh;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          load_n<WN>(x + (size_t)min(kb + j, K - 1) * T + col0, xr[0][j]);
+#pragma unroll
+          for (int b = 0; b < WN; ++b) xr[0][j][b] = kb + j < K ? xr[0][j][b] : 0.f;
+        }
+        if (SPLIT && !scaled) {
+          if (scales(xr[0])) return true;
+          scaled = true;
+        }
+        step(s, xr[0]);
+      }
+    }
+    if constexpr (SPLIT) {
+      if (scaled) {  // back to the operands' own scale
+#pragma unroll
+        for (int a = 0; a < WM; ++a)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x4 ir = *(const f32x4*)&inv_row[wave][32 * a + 8 * q + 4 * hh];
+#pragma unroll
+            for (int b = 0; b < WN; ++b) {
+              const float ib = 1.0f / sb[b];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[a][b][4 * q + e] = acc[a][b][4 * q + e] * ir[e] * ib;
+            }
+          }
+      }
+    }
+    return false;
+  };
+
+  // The waves' partial sums meet in LDS ([wave][a][b][q][lane], four rows
+  // each) and are added in wave order.  CHECK: if one is inf or NaN (or a
+  // wave could not split) nothing is stored and the result is false.
+  auto finish = [&](auto check_tag, bool bad) -> bool {
+    constexpr bool CHECK = decltype(check_tag)::value;
+    constexpr int UPT = (WM * 4 + KW - 1) / KW;  // (a, q) units per wave
+    __syncthreads();                             // the staging areas are free
+    f32x4* part = (f32x4*)lds + wave * (PART / 4);
+#pragma unroll
+    for (int a = 0; a < WM; ++a)
+#pragma unroll
+      for (int b = 0; b < WN; ++b)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          part[((a * WN + b) * 4 + q) * 64 + lane] =
+              f32x4{acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
+    __syncthreads();
+    f32x4 sum[UPT][WN];
+    float z = 0.f;
+#pragma unroll
+    for (int u = 0; u < UPT; ++u) {
+      const int aq = wave + KW * u;
+      if (aq >= WM * 4) break;
+      const f32x4* src = (const f32x4*)lds + ((aq >> 2) * WN * 4 + (aq & 3)) * 64 + lane;
+#pragma unroll
+      for (int b = 0; b < WN; ++b) {
+        f32x4 t = src[b * 256];
+#pragma unroll
+        for (int k = 1; k < KW; ++k) t += src[b * 256 + k * (PART / 4)];
+        sum[u][b] = t;
+        if (CHECK) z += t.x * 0.f + t.y * 0.f + (t.z * 0.f + t.w * 0.f);
+      }
+    }
+    if (CHECK && __syncthreads_or(bad || z != 0.f)) return false;
+#pragma unroll
+    for (int u = 0; u < UPT; ++u) {
+      const int aq = wave + KW * u;
+      if (aq >= WM * 4) break;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + 32 * (aq >> 2) + 8 * (aq & 3) + 4 * hh + e;
+        if (m >= M || nom >= T) continue;
+        float* dst = y + (size_t)m * T + col0;
+        if (WN > 1 && col0 == nom) {
+          typename FVec<WN == 1 ? 2 : WN>::T v;
+#pragma unroll
+          for (int b = 0; b < WN; ++b) v[b] = sum[u][b][e];
+          *(typename FVec<WN == 1 ? 2 : WN>::T*)dst = v;
+        } else {
+#pragma unroll
+          for (int b = 0; b < WN; ++b)
+            if (col0 + b >= nom) dst[b] = sum[u][b][e];
+        }
+      }
+    }
+    return true;
+  };
+  const bool bad = body(std::true_type{});
+  if (finish(std::true_type{}, bad)) return;
+  body(std::false_type{});
+  finish(std::false_type{}, false);
 }
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
+
+// The split GEMM's variants: tile, workgroups resident on a CU, and the model
+// of their time by which one is chosen, in us:
+//   2 + rounds of workgroups * (fixed + K / 1000 * (only round ? one : more)).
+// Fitted to 78 timed shapes (256 .. 14336 rows and k, 2 .. 4096 columns): the
+// choice is 0.2% off the best of the four on average, 7% at worst; always
+// taking 64x64 would cost 1.9x at 37 columns, always 32x32 2.2x at 1000.
+struct SplitVariant {
+  int bm, bn, per_cu;
+  float fixed, one, more;
+};
+constexpr SplitVariant kSplit[] = {
+    {32, 32, 1, 1.39f, 3.91f, 5.15f},    // 8 waves
+    {64, 64, 1, 3.51f, 7.56f, 9.86f},    // 8 waves
+    {64, 64, 2, 4.46f, 13.33f, 11.67f},  // 4 waves
+    {64, 128, 1, 5.57f, 11.78f, 11.37f}, // 4 waves
+};
 
 LinearPlan linear_plan(int M, int K, int T, const float* w, const float* x) {
   LinearPlan p{};
@@ -295,23 +544,38 @@ LinearPlan linear_plan(int M, int K, int T, const float* w, const float* x) {
     p.vec = (K % 4 == 0) && aligned16(w) && aligned16(x);
     p.wpr = M >= 2048 ? 1 : 4;
     p.grid_x = (M + 4 / p.wpr - 1) / (4 / p.wpr);
-    p.grid_y = 1;
-  } else {
-    p.gemv = false;
-    p.vec = (K % 4 == 0) && (T % 4 == 0) && aligned16(w) && aligned16(x);
-    const long long big = (long long)((M + 127) / 128) * ((T + 127) / 128);
-    p.tile = big >= 512 ? 128 : 64;
-    p.grid_x = (T + p.tile - 1) / p.tile;
-    p.grid_y = (M + p.tile - 1) / p.tile;
+    return p;
+  }
+  float best = 0.f;
+  const int cus = cu_count();
+  for (int v = 0; v < (int)(sizeof(kSplit) / sizeof(kSplit[0])); ++v) {
+    const SplitVariant& s = kSplit[v];
+    if (T < s.bn / 32) continue;  // a lane holds bn / 32 columns
+    const long long tm = ((long long)M + s.bm - 1) / s.bm, tn = ((long long)T + s.bn - 1) / s.bn;
+    const long long rounds = (tm * tn + (long long)cus * s.per_cu - 1) / ((long long)cus * s.per_cu);
+    const float t = 2.f + (float)rounds * (s.fixed + (rounds > 1 ? s.more : s.one) * (float)K * 1e-3f);
+    if (p.tiles_m == 0 || t < best) {
+      best = t;
+      p.variant = v;
+      p.tiles_m = (int)tm;
+      p.tiles_n = (int)tn;
+    }
   }
   return p;
+}
+
+template <int WM, int WN, int KW, int CK, int XD>
+static void launch_split(float* y, const float* x, const float* w, int K, int M, int T, const LinearPlan& p,
+                         hipStream_t stream) {
+  hipLaunchKernelGGL((linear_split_kernel<WM, WN, KW, CK, XD>), dim3((unsigned)p.tiles_m * (unsigned)p.tiles_n),
+                     dim3(64 * KW), 0, stream, w, x, y, M, K, T, p.tiles_m, p.tiles_n, WN == 4 ? 4 : 8);
 }
 
 hipError_t linear_col_launch(float* y, const float* x, const float* w, int K, int M, int T,
                              hipStream_t stream) {
   const LinearPlan p = linear_plan(M, K, T, w, x);
-  const dim3 grid(p.grid_x, p.grid_y), block(256);
   if (p.gemv) {
+    const dim3 grid(p.grid_x), block(256);
     if (p.wpr == 1) {
       if (p.vec) hipLaunchKernelGGL((linear_gemv_kernel<1, true>), grid, block, 0, stream, w, x, y, M, K);
       else hipLaunchKernelGGL((linear_gemv_kernel<1, false>), grid, block, 0, stream, w, x, y, M, K);
@@ -319,13 +583,13 @@ hipError_t linear_col_launch(float* y, const float* x, const float* w, int K, in
       if (p.vec) hipLaunchKernelGGL((linear_gemv_kernel<4, true>), grid, block, 0, stream, w, x, y, M, K);
       else hipLaunchKernelGGL((linear_gemv_kernel<4, false>), grid, block, 0, stream, w, x, y, M, K);
     }
-  } else if (p.tile == 128) {
-    if (p.vec) hipLaunchKernelGGL((linear_mfma_kernel<2, 2, 32, 1, true>), grid, block, 0, stream, w, x, y, M, K, T);
-    else hipLaunchKernelGGL((linear_mfma_kernel<2, 2, 32, 1, false>), grid, block, 0, stream, w, x, y, M, K, T);
-  } else {
-    if (p.vec) hipLaunchKernelGGL((linear_mfma_kernel<1, 1, 64, 2, true>), grid, dim3(512), 0, stream, w, x, y, M, K, T);
-    else hipLaunchKernelGGL((linear_mfma_kernel<1, 1, 64, 2, false>), grid, dim3(512), 0, stream, w, x, y, M, K, T);
+    return hipGetLastError();
   }
+  if ((long long)p.tiles_m * p.tiles_n > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+  if (p.variant == 0) launch_split<1, 1, 8, 64, 4>(y, x, w, K, M, T, p, stream);
+  else if (p.variant == 1) launch_split<2, 2, 8, 32, 2>(y, x, w, K, M, T, p, stream);
+  else if (p.variant == 2) launch_split<2, 2, 4, 32, 2>(y, x, w, K, M, T, p, stream);
+  else launch_split<2, 4, 4, 64, 2>(y, x, w, K, M, T, p, stream);
   return hipGetLastError();
 }
 
