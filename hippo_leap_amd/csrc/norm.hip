@@ -1,6 +1,6 @@
 // RMSNorm of the hidden state around the attention block, fp32 on the
 // reference's column-major activations:
-//   * rmsnorm_cols_kernel: gpuRmsnormCols (backends/naive.nim:2801-2843),
+//   * norm_cols_kernel: gpuRmsnormCols (backends/naive.nim:2801-2843),
 //     the norm in front of the Q/K/V projections (naive.nim:4063, 4095) and
 //     the final norm before the logits (naive.nim:5537):
 //     out[r, t] = x[r, t] * (1/sqrtf(sum_r x[r, t]^2 / dim + eps)) * w[r].
@@ -32,8 +32,8 @@ __device__ inline float block_sum(float v) {
   return (part[0] + part[1]) + (part[2] + part[3]);
 }
 
-// One column (seq_len == 1, or one workgroup per column when seq_len is
-// small): 256 threads stride over the rows.
+// One column (seq_len == 1), or one workgroup per column when seq_len is
+// small: 256 threads stride over the rows.
 __global__ __launch_bounds__(256) void rmsnorm_col_kernel(const float* __restrict__ x,
                                                           const float* __restrict__ w,
                                                           float* out, int dim, int seq, float eps) {
@@ -50,31 +50,58 @@ __global__ __launch_bounds__(256) void rmsnorm_col_kernel(const float* __restric
   }
 }
 
-// 64 adjacent columns per workgroup (lanes along t, coalesced), the four
-// waves splitting the rows; the column sums meet in LDS.
-__global__ __launch_bounds__(256) void rmsnorm_cols64_kernel(const float* __restrict__ x,
-                                                             const float* __restrict__ w,
-                                                             float* out, int dim, int seq,
-                                                             float eps) {
-  __shared__ float part[4][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int col = blockIdx.x * 64 + lane;
-  const bool live = col < seq;
-  float ss = 0.f;
-  if (live)
-    for (int r = wave; r < dim; r += 4) {
-      const float v = x[(size_t)r * seq + col];
-      ss += v * v;
-    }
-  part[wave][lane] = ss;
-  __syncthreads();
-  const float tot = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+// Columns of a prompt: a workgroup of 1024 threads takes CB columns, thread
+// (g, c) rows g, g + G, ... of column c, its first NR values kept in
+// registers between the two passes (all loads issued before the first is
+// used).  out may be x.
+//
+// Bound by the latency of one pass over few columns: the walk down a column
+// must be short, since seq / CB workgroups are all there are.  64 columns per
+// 256-thread workgroup (512 dependent-load rounds per thread at dim 2048, 5
+// workgroups at 301 columns) took 172 us for 2048 x 301; 8 columns: 9.1 us.
+// 16 columns (64-byte segments) from 2048 columns on, where the grid has a
+// workgroup for half of the CUs anyway (4096 x 4096: 51 us against 82 with 8;
+// 647 with 64).
+template <int CB, int NR>
+__global__ __launch_bounds__(1024) void norm_cols_kernel(const float* x, const float* __restrict__ w, float* out,
+                                                         int dim, int seq, float eps) {
+  constexpr int G = 1024 / CB;
+  __shared__ float part[16][CB];
+  const int c = threadIdx.x % CB, g = threadIdx.x / CB;
+  const int col = blockIdx.x * CB + c;
+  const size_t cc = min(col, seq - 1);
+  float v[NR], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NR; ++i) v[i] = x[(size_t)min(g + G * i, dim - 1) * seq + cc];
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+    if (g + G * i < dim) ss += v[i] * v[i];
+  for (int r0 = g + G * NR; r0 < dim; r0 += G * 8) {  // not kept; eight rows in flight
+    float t[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t[i] = x[(size_t)min(r0 + G * i, dim - 1) * seq + cc];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (r0 + G * i < dim) ss += t[i] * t[i];
+  }
+#pragma unroll
+  for (int o = CB; o < 64; o <<= 1) ss += __shfl_xor(ss, o, 64);
+  if ((threadIdx.x & 63) < CB) part[threadIdx.x >> 6][c] = ss;
+  __syncthreads();  // also: every read of the first pass before a store in place
+  float tot = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) tot += part[i][c];
+  if (col >= seq) return;
   const float inv = 1.0f / sqrtf(tot / (float)dim + eps);
-  if (live)
-    for (int r = wave; r < dim; r += 4) {
-      const size_t i = (size_t)r * seq + col;
-      out[i] = x[i] * inv * w[r];
-    }
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int r = g + G * i;
+    if (r < dim) out[(size_t)r * seq + cc] = v[i] * inv * w[r];
+  }
+  for (int r = g + G * NR; r < dim; r += G) {  // this thread's own rows
+    const size_t at = (size_t)r * seq + cc;
+    out[at] = x[at] * inv * w[r];
+  }
 }
 
 // x = xin + res (xin may be x), out = rmsnorm(x) * w (out may be xin: each
@@ -156,11 +183,14 @@ hipError_t rmsnorm_cols_launch(float* out, const float* x, const float* w, int d
   if (seq == 1 && vec4_ok(dim, x, w, out, out))
     hipLaunchKernelGGL(norm_vec4_kernel<false>, dim3(1), dim3(1024), 0, stream, const_cast<float*>(x), x,
                        nullptr, w, out, dim, eps);
-  else if (seq < 64)
+  else if (seq < 64)  // 4096 x 37: 9.4 us against 9.5, x 7: 6.8 against 7.8
     hipLaunchKernelGGL(rmsnorm_col_kernel, dim3(seq), dim3(256), 0, stream, x, w, out, dim, seq, eps);
+  else if (seq >= 2048)
+    hipLaunchKernelGGL((norm_cols_kernel<16, 32>), dim3((seq + 15) / 16), dim3(1024), 0, stream, x, w, out, dim, seq, eps);
+  else if (dim <= 2048)
+    hipLaunchKernelGGL((norm_cols_kernel<8, 16>), dim3((seq + 7) / 8), dim3(1024), 0, stream, x, w, out, dim, seq, eps);
   else
-    hipLaunchKernelGGL(rmsnorm_cols64_kernel, dim3((seq + 63) / 64), dim3(256), 0, stream, x, w,
-                       out, dim, seq, eps);
+    hipLaunchKernelGGL((norm_cols_kernel<8, 32>), dim3((seq + 7) / 8), dim3(1024), 0, stream, x, w, out, dim, seq, eps);
   return hipGetLastError();
 }
 

@@ -60,3 +60,21 @@ def test_residual_rmsnorm_misaligned(hl, orc):
     assert np.array_equal(xd.cpu().numpy(), xs)
     assert rel_err(out.cpu().numpy(), orc.rmsnorm(xs.reshape(1, dim), w, 1e-6).reshape(-1)) < TOL_F32
 
+
+@pytest.mark.parametrize("dim,T", [(2048, 301), (2049, 65), (4097, 71), (127, 66), (9001, 129), (96, 2048), (2050, 2063)])
+def test_rmsnorm_cols_of_a_prompt(hl, dim, T):
+    """The kernel that keeps a thread's rows in registers (T >= 64): around
+    its row groups, more rows than it keeps, both column counts, in place.
+    Bound: the sum of squares and three roundings, (dim / 64 + 16) 2^-24."""
+    from hippo_leap_amd import attention as A
+    print(f"rmsnorm_cols prompt dim={dim} T={T}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(dim + T)
+    x = torch.randn(dim, T, device="cuda", generator=g) * 3
+    w = torch.rand(dim, device="cuda", generator=g) + 0.5
+    ref = x.double() / torch.sqrt((x.double() ** 2).mean(0, keepdim=True) + 1e-5) * w.double()[:, None]
+    out = torch.full((dim * T + 32,), 7.5, device="cuda")
+    A.gpu_rmsnorm_cols(out, x, w, dim, T, 1e-5)
+    A.gpu_rmsnorm_cols(x, x, w, dim, T, 1e-5)
+    for got in (out[:dim * T].reshape(dim, T), x):
+        assert ((got.double() - ref).abs() / ref.abs().clamp_min(1e-30)).max().item() < (dim / 64 + 16) * 2.0 ** -24
+    assert bool((out[dim * T:] == 7.5).all())
