@@ -190,6 +190,24 @@ long long quant_row_bytes(int qtype, int K);
 hipError_t linear_quant_launch(float* y, const float* x, const void* w, int K, int M, int qtype,
                                hipStream_t stream);
 
+// The int8 matrix-core GEMV (linear_quant_i8.hip) over up to three matrices
+// of one type and width; pair: two matrices, y[0] = silu(w[0] n) * (w[1] n).
+// res: n = rmsnorm(x + res) * nrm and x + res goes to xsum (none of the
+// kernel's other buffers); otherwise n = x.  false: not its case.
+struct QuantI8Call {
+  int qtype, K, nmat;
+  bool pair;
+  const void* w[3];
+  float* y[3];
+  int rows[3];
+  const float* x;
+  const float* res;
+  const float* nrm;
+  float* xsum;
+  float eps;
+};
+bool linear_quant_i8_launch(const QuantI8Call& c, hipStream_t stream);
+
 // ---- RMSNorm of the hidden state (norm.hip) --------------------------------
 hipError_t rmsnorm_cols_launch(float* out, const float* x, const float* w, int dim, int seq,
                                float eps, hipStream_t stream);
@@ -215,11 +233,16 @@ bool linear_quant_pair_launch(int pair, float* y, float* y2, const float* x, con
 // Q, K and V projections of one x in one launch (false: run them apart).
 bool linear_quant_qkv_launch(float* yq, float* yk, float* yv, const float* x, const void* wq, const void* wk,
                              const void* wv, int K, int Mq, int Mkv, int qtype, hipStream_t stream);
-// xsum = x + res, then the fused gate/up/SiLU of rmsnorm(xsum) * nrm in one
-// launch (Q4_K on the matrix cores, K <= 8192); false when not applicable.
+// xsum = x + res, then the fused gate/up/SiLU of rmsnorm(xsum) * nrm (or
+// plain products of up to three matrices) in one launch on the matrix cores;
+// false when not applicable.
 bool linear_quant_gate_up_norm_launch(float* y, float* xsum, const float* x, const float* res, const float* nrm,
                                       float eps, const void* wg, const void* wu, int K, int M, int qtype,
                                       hipStream_t stream);
+
+bool linear_quant_norm_launch(int nmat, const void* const* w, float* const* y, const int* rows, int qtype, int K,
+                              float* xsum, const float* x, const float* res, const float* nrm, float eps,
+                              hipStream_t stream);
 
 // Sets the thread's hl_last_error() message (printf format); returns code.
 int set_error(int code, const char* fmt, ...);

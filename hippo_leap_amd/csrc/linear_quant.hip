@@ -1115,7 +1115,8 @@ __global__ __launch_bounds__(1024) void q4k_mfma_kernel(const uint8_t* __restric
   }
 }
 
-// The MFMA kernel pays for its x prologue (~2 us of latency before the
+// What the int8 kernel does not take (K < 2048 or > 16384, rows not on 16
+// bytes).  The MFMA kernel pays for its x prologue (~2 us of latency before the
 // first product) on matrices of 2^25 weights and more: 14336 x 4096 10.8 us
 // against 15.7, 4096 x 14336 14.2 against 17.0, but 4096 x 4096 8.3 against
 // 6.6 (kernel durations).  A fused pair streams both matrices behind one x
@@ -1178,6 +1179,50 @@ void launch_direct(const uint8_t* w, const float* x, float* y, int M, int K, hip
                      M, K, w2, y2, w3, y3, M2);
 }
 
+// The int8 matrix-core kernel (linear_quant_i8.hip) has 1.3-3 us more of
+// fixed cost than the direct kernel (x to digits, LDS stages) and streams
+// 4.2-6.3 TB/s where that reaches 2.2-3.6 (its VALU work per weight): it
+// takes over at 2^25 weights, a pair counting both matrices.  us, direct (or
+// q4k_mfma_kernel for Q4_K) -> int8:
+//                     Q4_K          Q5_K          Q6_K          Q8_0
+//   4096 x 4096       5.4 ->  6.6   5.8 ->  7.1   7.5 ->  8.5   7.3 ->  8.2
+//   2x 4096 x 4096    8.4 ->  8.3  10.2 ->  9.2  11.3 -> 11.5  12.1 -> 10.5
+//   2x 8192 x 2048    8.1 ->  7.6  12.6 ->  8.8  11.3 -> 10.6  12.3 -> 10.8
+//   4096 x 14336     12.1 -> 10.8  17.1 -> 13.4  18.0 -> 15.5  20.1 -> 15.2
+//   2x 14336 x 4096  16.0 -> 14.6  29.6 -> 17.8  32.8 -> 22.9  34.5 -> 22.6
+//   128256 x 2048    30.4 -> 27.6  81.2 -> 33.8  68.0 -> 42.4  68.8 -> 45.0
+// With the residual and RMSNorm folded in (two launches before, q4k_mfma's
+// own fold from 2^25), from 2^22 weights on: 2x 2048 x 2048 Q4_K 6.6 -> 5.5,
+// 2x 8192 x 2048 9.0 -> 8.5, 2x 14336 x 4096 16.8 -> 15.2.
+constexpr long long kI8Weights = 1LL << 25, kI8NormWeights = 1LL << 22;
+
+template <int QT>
+bool try_i8(bool pair, int nmat, const uint8_t* const* w, float* const* y, const int* rows, const float* x, int K,
+            hipStream_t stream) {
+  if constexpr (QT == HL_GGML_Q4_K || QT == HL_GGML_Q5_K || QT == HL_GGML_Q6_K || QT == HL_GGML_Q8_0) {
+    long long total = 0;
+    QuantI8Call c{};
+    for (int i = 0; i < nmat; ++i) {
+      total += (long long)rows[i] * K;
+      c.w[i] = w[i];
+      c.y[i] = y[i];
+      c.rows[i] = rows[i];
+    }
+    // Q6_K pays later (2x 4096 x 4096: 11.3 us either way), Q8_0 only from K =
+    // 4096 or 1.5 2^25 on (2x 6400 x 2816: 13.9 against 14.9).
+    if (total < kI8Weights || (QT == HL_GGML_Q6_K && total < 40000000) ||
+        (QT == HL_GGML_Q8_0 && K < 4096 && total < kI8Weights * 3 / 2))
+      return false;
+    c.qtype = QT;
+    c.K = K;
+    c.nmat = nmat;
+    c.pair = pair;
+    c.x = x;
+    return linear_quant_i8_launch(c, stream);
+  }
+  return false;
+}
+
 template <int QT, int KS>
 void launch_direct_r(const uint8_t* w, const float* x, float* y, int M, int K, hipStream_t stream) {
   constexpr bool r4 = QT != 12 && QT != 13 && QT != 14;  // the K-quants at four rows: ~200+ VGPRs
@@ -1191,6 +1236,7 @@ void launch_direct_plan(const uint8_t* w, const float* x, float* y, int M, int K
   // Split a row's blocks over four waves when each gets a step: more waves
   // and loads in flight for decode-sized M.  (A two-way split of 2-3 steps
   // measured slower than none: Q4_K 4096x4096 5.5 -> 7.2 us.)
+  if (try_i8<QT>(false, 1, &w, &y, &M, x, K, stream)) return;
   if constexpr (QT == 12) {
     if (q4k_mfma_pays(M, K) && launch_q4k_mfma<0>(w, x, y, M, K, stream)) return;
   }
@@ -1217,6 +1263,10 @@ bool launch_pair_qt(const uint8_t* w, const uint8_t* w2, const float* x, float* 
                   (QT == 1 ? (a & 15) == 0 : (QT == 12 || QT == 13) ? (a & 15) == 0
                    : QT == 10 ? (a & 3) == 0 : (a & 1) == 0);
   if (!ok) return false;
+  const uint8_t* const ws[2] = {w, w2};
+  float* const ys[2] = {y, y2};
+  const int rows[2] = {M, M};
+  if (try_i8<QT>(PAIR == 1, 2, ws, ys, rows, x, K, stream)) return true;
   if constexpr (QT == 12) {
     if (q4k_mfma_pays(2 * M, K) && launch_q4k_mfma<PAIR>(w, x, y, M, K, stream, w2, y2)) return true;
   }
@@ -1351,6 +1401,10 @@ bool launch_qkv_qt(const uint8_t* wq, const uint8_t* wk, const uint8_t* wv, cons
                   (QT == 1 ? (a & 15) == 0 : (QT == 12 || QT == 13) ? (a & 15) == 0
                    : QT == 10 ? (a & 3) == 0 : (a & 1) == 0);
   if (!ok) return false;
+  const uint8_t* const ws[3] = {wq, wk, wv};
+  float* const ys[3] = {yq, yk, yv};
+  const int rows[3] = {Mq, Mkv, Mkv};
+  if (try_i8<QT>(false, 3, ws, ys, rows, x, K, stream)) return true;
   if constexpr (QT == 12) {
     if (q4k_mfma_pays(Mq, K) || q4k_mfma_pays(Mkv, K)) return false;
   }
@@ -1361,20 +1415,38 @@ bool launch_qkv_qt(const uint8_t* wq, const uint8_t* wk, const uint8_t* wv, cons
   return true;
 }
 
-// Residual + RMSNorm folded into the fused gate/up/SiLU GEMV (Q4_K on the
-// matrix cores, K <= 8192): xsum = x + res; y = silu(G n) * (U n) with
-// n = rmsnorm(xsum) * nrm.  false: not this kernel's case (the caller runs
-// the norm and the pair separately).
+// Residual + RMSNorm folded into the fused gate/up/SiLU GEMV on the matrix
+// cores: xsum = x + res; y = silu(G n) * (U n) with n = rmsnorm(xsum) * nrm.
+// false: not these kernels' case (the caller runs the norm and the pair
+// separately).
 bool linear_quant_gate_up_norm_launch(float* y, float* xsum, const float* x, const float* res, const float* nrm,
                                       float eps, const void* wg, const void* wu, int K, int M, int qtype,
                                       hipStream_t stream) {
   const uintptr_t v = (uintptr_t)x | (uintptr_t)res | (uintptr_t)nrm | (uintptr_t)xsum;
   const uintptr_t a = (uintptr_t)wg | (uintptr_t)wu;
-  if (qtype != HL_GGML_Q4_K || M <= 0 || K <= 0 || K % 256 || K > 8192 || (v & 15) || (a & 15) ||
-      !q4k_mfma_pays(2 * M, K))
-    return false;
+  if (M <= 0 || K <= 0 || K % 256 || (v & 15) || (a & 15)) return false;
+  if (2LL * M * K >= kI8NormWeights) {
+    const QuantI8Call c{qtype, K, 2, true, {wg, wu}, {y}, {M, M}, x, res, nrm, xsum, eps};
+    if (linear_quant_i8_launch(c, stream)) return true;
+  }
+  if (qtype != HL_GGML_Q4_K || K > 8192 || !q4k_mfma_pays(2 * M, K)) return false;
   return launch_q4k_mfma<1, true>((const uint8_t*)wg, x, y, M, K, stream, (const uint8_t*)wu, nullptr, res, nrm,
                                   xsum, eps);
+}
+
+// The same over up to three matrices of one type: y[i] = w[i] n.
+bool linear_quant_norm_launch(int nmat, const void* const* w, float* const* y, const int* rows, int qtype, int K,
+                              float* xsum, const float* x, const float* res, const float* nrm, float eps,
+                              hipStream_t stream) {
+  QuantI8Call c{qtype, K, nmat, false, {}, {}, {}, x, res, nrm, xsum, eps};
+  long long total = 0;
+  for (int i = 0; i < nmat; ++i) {
+    c.w[i] = w[i];
+    c.y[i] = y[i];
+    c.rows[i] = rows[i];
+    total += (long long)rows[i] * K;
+  }
+  return total >= kI8NormWeights && linear_quant_i8_launch(c, stream);
 }
 
 bool linear_quant_qkv_launch(float* yq, float* yk, float* yv, const float* x, const void* wq, const void* wk,
