@@ -7,9 +7,11 @@
 // Everything stays on the device between steps: the token is read from and
 // the next token written to device memory, so consecutive steps chain
 // without a host round trip.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <utility>
 
 #include "common.h"
 #include "launch.h"
@@ -211,40 +213,110 @@ static bool qkv_launch(float* q, float* k, float* v, const float* x, const hl_la
     if (rc_ != HL_OK) return rc_; \
   } while (0)
 
-// The FFN half of a decode layer after attention's O projection in tmp0:
-// residual + ffn norm, gate/up, SiLU * up, down, residual + the next
-// layer's norm (or the plain residual after the last layer).
-static int decode_ffn(const hl_model_desc* m, int l, float* x, float* x_norm, float* tmp0, float* tmp1, float* tmp2,
-                      void* stream) {
-  const hl_layer_desc& L = m->layers[l];
-  const int E = m->n_emb;
-  const float eps = m->rms_eps;
-  // Q4_K gate/up on the matrix cores takes the residual + norm into its own
-  // x prologue; the sum then sits in x_norm until the next residual moves it
-  // back to x.
-  const bool folded = L.w_gate_type == L.w_up_type &&
-                      linear_quant_gate_up_norm_launch(tmp2, x_norm, x, tmp0, L.ffn_norm, eps, L.w_gate, L.w_up, E,
-                                                       m->n_ff, L.w_gate_type, (hipStream_t)stream);
-  if (folded) {
-    if (hipGetLastError() != hipSuccess) return set_error(HL_EHIP, "fused norm gate/up launch failed");
-  } else {
-    HL_TRY(hl_gpu_residual_rmsnorm(x_norm, x, tmp0, L.ffn_norm, E, eps, stream));
-    if (!pair_launch(1, tmp2, nullptr, x_norm, L.w_gate, L.w_up, L.w_gate_type, L.w_up_type, E, m->n_ff, stream)) {
-      HL_TRY(linear_t(tmp0, x_norm, L.w_gate, L.w_gate_type, E, m->n_ff, 1, stream));
-      HL_TRY(linear_t(tmp1, x_norm, L.w_up, L.w_up_type, E, m->n_ff, 1, stream));
-      HL_TRY(hl_gpu_silu_mul(tmp2, tmp0, tmp1, m->n_ff, stream));
-    }
-  }
-  HL_TRY(linear_t(tmp0, tmp2, L.w_down, L.w_down_type, m->n_ff, E, 1, stream));
-  const float* xs = folded ? x_norm : x;  // the residual stream
-  if (l + 1 < m->n_layer) {
-    if (residual_rmsnorm_from_launch(x_norm, x, xs, tmp0, m->layers[l + 1].attn_norm, E, eps, (hipStream_t)stream) !=
-        hipSuccess)
+// The buffers of a decode step between its launches.  The residual stream is
+// in S (x or x_norm), the projection not yet added to it in res (null before
+// the first layer).  A launch that folds the addition and the norm into its
+// own x prologue writes the sum to the other of the two, T, which no
+// workgroup of it reads.  A one-column norm is a launch of one workgroup that
+// nothing overlaps (4.5 us); the fold costs its GEMV about 1 us.  Llama-3.2-1B
+// shapes in Q4_K at 2K columns: 637 us a token with the fold in gate/up only,
+// 612 with it in Q/K/V and the head too.
+struct DecodeFlow {
+  const hl_model_desc* m;
+  float *x, *xn, *t0, *t1, *t2;
+  void* stream;
+  float* S;
+  float* T;
+  const float* res;
+  float *q, *k, *v, *att, *o;  // this layer's projections, attention output and O projection
+
+  DecodeFlow(const hl_model_desc* m_, float* x_, float* xn_, float* t0_, float* t1_, float* t2_, void* st)
+      : m(m_), x(x_), xn(xn_), t0(t0_), t1(t1_), t2(t2_), stream(st), S(x_), T(xn_), res(nullptr) {}
+
+  // x = S + res, xn = rmsnorm(x) * weight, by a launch of its own.
+  int norm(const float* weight) {
+    if (!res) return hl_gpu_rmsnorm_cols(xn, x, weight, m->n_emb, 1, m->rms_eps, stream);
+    if (S == x) return hl_gpu_residual_rmsnorm(xn, x, res, weight, m->n_emb, m->rms_eps, stream);
+    if (residual_rmsnorm_from_launch(xn, x, S, res, weight, m->n_emb, m->rms_eps, (hipStream_t)stream) != hipSuccess)
       return set_error(HL_EHIP, "residual rmsnorm launch failed");
+    S = x;
+    T = xn;
     return HL_OK;
   }
-  return hl_gpu_add(x, xs, tmp0, E, stream);
-}
+  bool folded(bool launched) {
+    if (launched) std::swap(S, T);
+    return launched;
+  }
+
+  // Norm and Q/K/V projections of layer l.  Folded, res (in t0) is read by
+  // the launch that writes q, so q goes behind it in t0; the attention output
+  // then takes the place of res and the O projection that of k.
+  int qkv(int l) {
+    const hl_layer_desc& L = m->layers[l];
+    const int E = m->n_emb, qdim = m->n_head * m->head_dim, kvdim = m->n_head_kv * m->head_dim;
+    const int at = (std::max(E, qdim) + 63) / 64 * 64;
+    if (res && L.wq_type != 0 && L.wq_type == L.wk_type && L.wq_type == L.wv_type &&
+        std::max({E, qdim, m->n_ff}) >= at + qdim && std::max(kvdim, m->n_ff) >= E) {
+      const void* const ws[3] = {L.wq, L.wk, L.wv};
+      float* const ys[3] = {t0 + at, t1, t2};
+      const int rows[3] = {qdim, kvdim, kvdim};
+      if (folded(linear_quant_norm_launch(3, ws, ys, rows, L.wq_type, E, T, S, res, L.attn_norm, m->rms_eps,
+                                          (hipStream_t)stream))) {
+        q = t0 + at, k = t1, v = t2, att = t0, o = t1;
+        return hipGetLastError() == hipSuccess ? HL_OK : set_error(HL_EHIP, "fused norm Q/K/V launch failed");
+      }
+    }
+    HL_TRY(norm(L.attn_norm));
+    q = t0, k = t1, v = t2, att = xn, o = t0;
+    if (qkv_launch(q, k, v, xn, L, E, qdim, kvdim, stream)) return HL_OK;
+    HL_TRY(linear_t(q, xn, L.wq, L.wq_type, E, qdim, 1, stream));
+    if (pair_launch(2, k, v, xn, L.wk, L.wv, L.wk_type, L.wv_type, E, kvdim, stream)) return HL_OK;
+    HL_TRY(linear_t(k, xn, L.wk, L.wk_type, E, kvdim, 1, stream));
+    return linear_t(v, xn, L.wv, L.wv_type, E, kvdim, 1, stream);
+  }
+
+  // O projection, then the FFN half: residual + ffn norm, gate/up, SiLU * up,
+  // down.
+  int rest(int l) {
+    const hl_layer_desc& L = m->layers[l];
+    const int E = m->n_emb, qdim = m->n_head * m->head_dim;
+    HL_TRY(linear_t(o, att, L.wo, L.wo_type, qdim, E, 1, stream));
+    res = o;
+    if (L.w_gate_type == L.w_up_type &&
+        folded(linear_quant_gate_up_norm_launch(t2, T, S, res, L.ffn_norm, m->rms_eps, L.w_gate, L.w_up, E, m->n_ff,
+                                                L.w_gate_type, (hipStream_t)stream))) {
+      if (hipGetLastError() != hipSuccess) return set_error(HL_EHIP, "fused norm gate/up launch failed");
+    } else {
+      HL_TRY(norm(L.ffn_norm));
+      if (!pair_launch(1, t2, nullptr, xn, L.w_gate, L.w_up, L.w_gate_type, L.w_up_type, E, m->n_ff, stream)) {
+        HL_TRY(linear_t(t0, xn, L.w_gate, L.w_gate_type, E, m->n_ff, 1, stream));
+        HL_TRY(linear_t(t1, xn, L.w_up, L.w_up_type, E, m->n_ff, 1, stream));
+        HL_TRY(hl_gpu_silu_mul(t2, t0, t1, m->n_ff, stream));
+      }
+    }
+    HL_TRY(linear_t(t0, t2, L.w_down, L.w_down_type, m->n_ff, E, 1, stream));
+    res = t0;
+    return HL_OK;
+  }
+
+  // Final residual and norm, output projection, greedy token.
+  int head(float* logits, int32_t* next) {
+    const void* const ws[1] = {m->output};
+    float* const ys[1] = {logits};
+    const uintptr_t lo = (uintptr_t)logits, hi = lo + (size_t)m->n_vocab * 4;
+    const auto apart = [&](const float* p) { return (uintptr_t)(p + m->n_emb) <= lo || hi <= (uintptr_t)p; };
+    // logits may lie in the scratch that the unfolded launches are done with
+    if (m->output_type != 0 && apart(S) && apart(T) && apart(res) &&
+        folded(linear_quant_norm_launch(1, ws, ys, &m->n_vocab, m->output_type, m->n_emb, T, S, res, m->output_norm,
+                                        m->rms_eps, (hipStream_t)stream))) {
+      if (hipGetLastError() != hipSuccess) return set_error(HL_EHIP, "fused norm output projection launch failed");
+    } else {
+      HL_TRY(norm(m->output_norm));
+      HL_TRY(linear_t(logits, xn, m->output, m->output_type, m->n_emb, m->n_vocab, 1, stream));
+    }
+    return hl_argmax_async(logits, m->n_vocab, next, stream);
+  }
+};
 
 // The gpuAttentionDecode call of the reference's step for layer l (fp32
 // caches of the model descriptor).
@@ -279,33 +351,24 @@ int hl_forward_decode_token(const hl_model_desc* m, const hl_decode_scratch* s,
     dropin_args(a, m, l, s->tmp0, s->x_norm, pos + 1);
     HL_TRY(check_decode_args(&a));
   }
-  const int E = m->n_emb, D = m->head_dim, qdim = m->n_head * D, kvdim = m->n_head_kv * D;
+  const int D = m->head_dim, kvdim = m->n_head_kv * D;
   const int rd = rope_dim_of(m);
   const float eps = m->rms_eps;
   HL_TRY(hl_set_rope_theta(rd, m->rope_base));
-  HL_TRY(hl_gpu_embedding(s->x, m->tok_emb, token_dev, E, 1, m->n_vocab, stream));
-  HL_TRY(hl_gpu_rmsnorm_cols(s->x_norm, s->x, m->layers[0].attn_norm, E, 1, eps, stream));
+  HL_TRY(hl_gpu_embedding(s->x, m->tok_emb, token_dev, m->n_emb, 1, m->n_vocab, stream));
+  DecodeFlow f(m, s->x, s->x_norm, s->tmp0, s->tmp1, s->tmp2, stream);
   for (int l = 0; l < m->n_layer; ++l) {
     const hl_layer_desc& L = m->layers[l];
-    if (!qkv_launch(s->tmp0, s->tmp1, s->tmp2, s->x_norm, L, E, qdim, kvdim, stream)) {
-      HL_TRY(linear_t(s->tmp0, s->x_norm, L.wq, L.wq_type, E, qdim, 1, stream));
-      if (!pair_launch(2, s->tmp1, s->tmp2, s->x_norm, L.wk, L.wv, L.wk_type, L.wv_type, E, kvdim, stream)) {
-        HL_TRY(linear_t(s->tmp1, s->x_norm, L.wk, L.wk_type, E, kvdim, 1, stream));
-        HL_TRY(linear_t(s->tmp2, s->x_norm, L.wv, L.wv_type, E, kvdim, 1, stream));
-      }
-    }
-    if (L.q_norm) HL_TRY(hl_gpu_qk_norm(s->tmp0, L.q_norm, m->n_head, D, eps, stream));
-    if (L.k_norm) HL_TRY(hl_gpu_qk_norm(s->tmp1, L.k_norm, m->n_head_kv, D, eps, stream));
-    HL_TRY(hl_gpu_rope_qk_decode(s->tmp0, s->tmp1, m->n_head, m->n_head_kv, D, rd, m->rope_base, pos, stream));
-    HL_TRY(hl_gpu_store_kv_pair(L.k_cache, s->tmp1, L.v_cache, s->tmp2, kvdim, 1, m->max_len, pos, stream));
-    HL_TRY(hl_gpu_attention_decode(s->x_norm, s->tmp0, L.k_cache, L.v_cache, m->n_head, m->n_head_kv,
+    HL_TRY(f.qkv(l));
+    if (L.q_norm) HL_TRY(hl_gpu_qk_norm(f.q, L.q_norm, m->n_head, D, eps, stream));
+    if (L.k_norm) HL_TRY(hl_gpu_qk_norm(f.k, L.k_norm, m->n_head_kv, D, eps, stream));
+    HL_TRY(hl_gpu_rope_qk_decode(f.q, f.k, m->n_head, m->n_head_kv, D, rd, m->rope_base, pos, stream));
+    HL_TRY(hl_gpu_store_kv_pair(L.k_cache, f.k, L.v_cache, f.v, kvdim, 1, m->max_len, pos, stream));
+    HL_TRY(hl_gpu_attention_decode(f.att, f.q, L.k_cache, L.v_cache, m->n_head, m->n_head_kv,
                                    D, pos + 1, m->max_len, stream));
-    HL_TRY(linear_t(s->tmp0, s->x_norm, L.wo, L.wo_type, qdim, E, 1, stream));
-    HL_TRY(decode_ffn(m, l, s->x, s->x_norm, s->tmp0, s->tmp1, s->tmp2, stream));
+    HL_TRY(f.rest(l));
   }
-  HL_TRY(hl_gpu_rmsnorm_cols(s->x_norm, s->x, m->output_norm, E, 1, eps, stream));
-  HL_TRY(linear_t(logits, s->x_norm, m->output, m->output_type, E, m->n_vocab, 1, stream));
-  return hl_argmax_async(logits, m->n_vocab, next_token_dev, stream);
+  return f.head(logits, next_token_dev);
 }
 
 // ---------------------------------------------------------------------------
@@ -546,31 +609,19 @@ int hl_forward_decode(const hl_model_desc* m, hl_kv_cache_desc* c, const hl_forw
   }
   HL_TRY(check_workspace(s, decode_region_bytes(m, c)));
 
-  const int E = m->n_emb, qdim = m->n_head * m->head_dim, kvdim = m->n_head_kv * m->head_dim;
-  const float eps = m->rms_eps;
-  HL_TRY(hl_gpu_embedding(s->x, m->tok_emb, token_dev, E, 1, m->n_vocab, stream));
-  HL_TRY(hl_gpu_rmsnorm_cols(s->x_norm, s->x, m->layers[0].attn_norm, E, 1, eps, stream));
+  HL_TRY(hl_gpu_embedding(s->x, m->tok_emb, token_dev, m->n_emb, 1, m->n_vocab, stream));
+  DecodeFlow f(m, s->x, s->x_norm, s->tmp0, s->tmp1, s->tmp2, stream);
   for (int l = 0; l < m->n_layer; ++l) {
-    const hl_layer_desc& L = m->layers[l];
-    if (!qkv_launch(s->tmp0, s->tmp1, s->tmp2, s->x_norm, L, E, qdim, kvdim, stream)) {
-      HL_TRY(linear_t(s->tmp0, s->x_norm, L.wq, L.wq_type, E, qdim, 1, stream));
-      if (!pair_launch(2, s->tmp1, s->tmp2, s->x_norm, L.wk, L.wv, L.wk_type, L.wv_type, E, kvdim, stream)) {
-        HL_TRY(linear_t(s->tmp1, s->x_norm, L.wk, L.wk_type, E, kvdim, 1, stream));
-        HL_TRY(linear_t(s->tmp2, s->x_norm, L.wv, L.wv_type, E, kvdim, 1, stream));
-      }
-    }
+    HL_TRY(f.qkv(l));
     // qk-norm + RoPE + the cache write at pos + attention over pos + 1
     // columns (naive.nim:4697-4717): one launch for fp16/bf16/fp8 caches
     hl_rope_store_args r;
     hl_decode_args a;
-    step_args(r, a, m, c, l, s->tmp0, s->tmp1, s->tmp2, s->x_norm, pos);
+    step_args(r, a, m, c, l, f.q, f.k, f.v, f.att, pos);
     HL_TRY(hl_decode_step(&r, &a, s->workspace, decode_region_bytes(m, c), stream));
-    HL_TRY(linear_t(s->tmp0, s->x_norm, L.wo, L.wo_type, qdim, E, 1, stream));
-    HL_TRY(decode_ffn(m, l, s->x, s->x_norm, s->tmp0, s->tmp1, s->tmp2, stream));
+    HL_TRY(f.rest(l));
   }
-  HL_TRY(hl_gpu_rmsnorm_cols(s->x_norm, s->x, m->output_norm, E, 1, eps, stream));
-  HL_TRY(linear_t(logits, s->x_norm, m->output, m->output_type, E, m->n_vocab, 1, stream));
-  HL_TRY(hl_argmax_async(logits, m->n_vocab, next_token_dev, stream));
+  HL_TRY(f.head(logits, next_token_dev));
   c->cur_len = pos + 1;
   return HL_OK;
 }

@@ -183,6 +183,37 @@ def test_forward_decode_token_norm_folded_into_gate_up(hl, orc, n_emb, n_ff):
         m.tokens[0] = tok
 
 
+# Residual + norm folded into the Q/K/V launch (3072 x 2048) and the output
+# projection (2100 x 2048): one type each, scratch wide enough for q behind
+# the residual (n_ff >= 2 n_emb); at 4032 it is not and only the head folds.
+# logits in tmp0 (allowed, the unfolded head is done with it) must not fold.
+@pytest.mark.parametrize("qtype,n_ff,logits_in_tmp0", [(8, 4096, False), (12, 4352, False), (13, 4096, False),
+                                                       (14, 4096, False), (8, 4032, False), (8, 4096, True)])
+def test_forward_decode_norm_folded_into_qkv_and_head(hl, orc, qtype, n_ff, logits_in_tmp0):
+    from hippo_leap_amd.model import DenseModel
+    print(f"decode model: norm folded into Q/K/V and head, type {qtype} n_ff {n_ff}", flush=True)
+    cfg = dict(CFG_WIDE, n_layer=3, n_ff=n_ff, n_vocab=2100)
+    types = {"wq": qtype, "wk": qtype, "wv": qtype, "wo": 8, "w_gate": 8, "w_up": 8, "w_down": 8, "output": qtype}
+    dev, ref = _build(orc, cfg, types, False, 173)
+    m = DenseModel(torch, cfg, dev["tok_emb"], dev["output_norm"], dev["output"], dev["output_type"], dev["layers"])
+    if logits_in_tmp0:
+        m.logits = m.fbufs[2][:cfg["n_vocab"]]
+    tok = 9
+    for pos in range(3):
+        m.tokens[0] = tok
+        m.decode()
+        torch.cuda.synchronize()
+        logits, nxt = m.logits.cpu().numpy(), int(m.tokens[1].item())
+        ref_logits = _oracle_step(orc, cfg, ref, tok, pos)
+        assert rel_err(logits, ref_logits) < TOL_F32, f"step {pos}"
+        assert nxt == orc.argmax(logits)
+        if not logits_in_tmp0:  # the descriptor's own caches, same step
+            m.step(pos)
+            torch.cuda.synchronize()
+            assert rel_err(m.logits.cpu().numpy(), ref_logits) < TOL_F32, f"step {pos}"
+        tok = nxt
+
+
 def test_forward_decode_token_rope_dim_zero(hl, orc):
     """rope_dim 0 means the whole head, as the reference's ropeDim =
     headDim when the model file has no rope dimension (naive.nim:3979)."""
