@@ -164,15 +164,26 @@ int prefill_mfma_tpad(int seq_len);
 
 // ---- fp32 linear layer (linear.hip) ----------------------------------------
 // Y[M, T] = W[M, K] . X[K, T]: GEMV for T == 1, GEMM on split operands otherwise.
-struct LinearPlan {
-  bool gemv;
-  bool vec;      // GEMV: 16-byte loads (K % 4 == 0, aligned w, x)
-  int wpr;       // GEMV: waves per row (1, or 4 when M is small)
-  int grid_x;    // GEMV
-  int variant;   // GEMM: index into the split GEMM's variants
-  int tiles_m, tiles_n;
+// One GEMM launch over up to three matrices and the same X (T >= 2): y[i] =
+// w[i] X; with res (one matrix; may be y[0]) y[0] = res + w[0] X; with pair
+// y[0] = silu(w[0] X) * (w[1] X), rows[0] of each.
+struct LinearCall {
+  int nmat;
+  const float* w[3];
+  float* y[3];
+  int rows[3];
+  const float* x;
+  const float* res;
+  bool pair;
+  int K, T;
 };
-LinearPlan linear_plan(int M, int K, int T, const float* w, const float* x);
+struct LinearPlan {
+  int variant;  // index into the GEMM's variants
+  int tiles_m, tiles_n;
+  int tend[2];  // row tiles up to and including the first and second matrix
+};
+LinearPlan linear_plan(const LinearCall& c);
+hipError_t linear_cols_launch(const LinearCall& c, hipStream_t stream);
 hipError_t linear_col_launch(float* y, const float* x, const float* w, int K, int M, int T,
                              hipStream_t stream);
 

@@ -120,9 +120,10 @@ __global__ __launch_bounds__(256) void linear_gemv_kernel(const float* __restric
 //
 // s brings the largest magnitude of the first 16 k that a wave meets into
 // [64, 128): the absolute error is then 2^-31 of it, and later elements may
-// be 2^9 times larger.  One above that, an inf or a NaN makes a partial sum inf or NaN, and the workgroup then computes its
-// tile once more with fp32 MFMAs (body<false>), so that inf and NaN come out
-// as fp32 arithmetic gives them.  A row or column whose first 16 elements are
+// be 2^9 times larger.  One above that, an inf or a NaN makes a partial sum
+// inf or NaN, and the workgroup then computes its tile once more with fp32
+// MFMAs (body<false>), so that inf and NaN come out as fp32 arithmetic gives
+// them.  A row or column whose first 16 elements are
 // zero is scanned for its largest element instead.
 //
 // The KW waves of a workgroup share one (32 WM) x (32 WN) output tile and
@@ -135,18 +136,28 @@ __global__ __launch_bounds__(256) void linear_gemv_kernel(const float* __restric
 // column blocks, and neither K nor T nor an address has to be a multiple of
 // anything.  The splits cost 2 (multiply) + 2 (v_cvt_pk_f16_f32) + 4
 // (v_fma_mix_f32) + 2 cycles per element and lane; v_fma_mixlo_f16, which
-// would take two instructions, measured 8 cycles each.
+// would take two instructions, measured 8 cycles each.  The splits of the next
+// column block and of the next step's rows stand between the MFMAs of this
+// one: 3 to 5% over splitting a block and then multiplying it (14336 x 4096,
+// 1000: 481 -> 464 us; 4096 x 14336: 459 -> 434; 4096 x 4096, 128: 34.2 -> 31.5).
+//
+// A launch takes up to three matrices on the same X, a residual to add, or
+// gate and up with SiLU * up on the sums: a prompt's layers then need four
+// GEMM launches for ten kernels, tiles of small matrices share a round, and
+// the sums of gate and up never go to memory.  Llama-3.2-1B shapes, 301
+// tokens, a whole prefill: 6.17 -> 5.46 ms (Q/K/V 51 -> 28 us a layer, gate,
+// up and SiLU 131 -> 105, the two additions 10 -> 0).
 //
 // What bounds it: bytes into the CUs on the small tiles (128 B per k of a
 // 64x64 tile from L2; the prefetch depth did not matter), the matrix cores
 // at three products on 64x128 tiles.  Before: fp32 MFMAs on 128x128 tiles
 // staged through LDS, scalar loads whenever K or T was no multiple of 4.
 //   M x K, T              before      now
-//   4096 x 4096,    37    130 us     20.7   (32x32 tiles)
-//   2048 x 2048,   301     76        23     (64x64)
-//   2048 x 8192,   301    267        70     (64x64)
-//   14336 x 4096, 1000   1080       479     (64x128: 245 TFLOP/s)
-//   4096 x 4096,  4096   1044       521     (64x128: 264 TFLOP/s)
+//   4096 x 4096,    37    130 us     19.9   (32x32 tiles)
+//   2048 x 2048,   301     76        20.4   (64x64)
+//   2048 x 8192,   301    267        62     (64x64)
+//   14336 x 4096, 1000   1080       464     (64x128: 253 TFLOP/s)
+//   4096 x 4096,  4096   1044       522     (64x128: 263 TFLOP/s)
 // Measured and not kept: x loads four steps ahead (no change), 64-k chunks on
 // 64x64 tiles (17% slower), sixteen waves (slower), 128x64 and 128x128 tiles.
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -178,15 +189,24 @@ __device__ __forceinline__ float split_rest(float x, float s, uint32_t hi) {
 __device__ __forceinline__ uint32_t pack_f16(float a, float b) {
   return __builtin_bit_cast(uint32_t, f16x2{(_Float16)a, (_Float16)b});
 }
-__device__ __forceinline__ void split8(const float* v, float s, f16x8& hi, f16x8& lo) {
-  u32x4 h, l;
+__device__ __forceinline__ void split2(float v0, float v1, float s, uint32_t& hi, uint32_t& lo) {
+  hi = pack_f16(v0 * s, v1 * s);
+  lo = pack_f16(split_rest<0>(v0, s, hi), split_rest<1>(v1, s, hi));
+}
+struct Split8 {
+  u32x4 hi, lo;
+};
+__device__ __forceinline__ f16x8 as_f16(const u32x4& v) { return __builtin_bit_cast(f16x8, v); }
+__device__ __forceinline__ Split8 split8(const float* v, float s) {
+  Split8 r;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) h[j] = pack_f16(v[2 * j] * s, v[2 * j + 1] * s);
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    l[j] = pack_f16(split_rest<0>(v[2 * j], s, h[j]), split_rest<1>(v[2 * j + 1], s, h[j]));
-  hi = __builtin_bit_cast(f16x8, h);
-  lo = __builtin_bit_cast(f16x8, l);
+  for (int j = 0; j < 4; ++j) {
+    uint32_t h, l;
+    split2(v[2 * j], v[2 * j + 1], s, h, l);
+    r.hi[j] = h;
+    r.lo[j] = l;
+  }
+  return r;
 }
 
 // The power of two that brings magnitude m into [64, 128) (1 for m = 0).  bad:
@@ -205,12 +225,22 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// group_m: tiles are walked group_m row tiles at a time, row tiles fastest.
-template <int WM, int WN, int KW, int CK, int XD>
-__global__ __launch_bounds__(64 * KW) void linear_split_kernel(const float* __restrict__ w,
-                                                               const float* __restrict__ x,
-                                                               float* __restrict__ y, int M, int K, int T,
-                                                               int tiles_m, int tiles_n, int group_m) {
+struct SplitArgs {
+  const float* w[3];
+  float* y[3];
+  int rows[3];
+  int tend[2];  // row tiles up to and including the first and second matrix
+  const float* x;
+  const float* res;  // added to y[0] (may be y[0]); null: none
+  int K, T, tiles_m, tiles_n;
+  int group_m;  // tiles are walked group_m row tiles at a time, row tiles fastest
+};
+
+// PAIR: w[0] and w[1] are gate and up, y[0] = silu(gate x) * (up x): each 32
+// rows of a tile are 16 of gate and the same 16 of up, which meet in one lane
+// of the final sums.  Otherwise the row tiles run over the matrices in order.
+template <int WM, int WN, int KW, int CK, int XD, bool PAIR>
+__global__ __launch_bounds__(64 * KW) void linear_split_kernel(SplitArgs p) {
   constexpr int ST = CK / 16;            // 16-k steps per chunk
   constexpr int BM = 32 * WM, BN = 32 * WN;
   constexpr int C16 = CK / 4;            // 16-byte pieces per staged row
@@ -228,24 +258,35 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(const float* __re
 
   // Each XCD (workgroup id mod 8) walks its own contiguous run of tiles, so
   // that its L2 serves the rows and columns its workgroups share.
-  const int total = tiles_m * tiles_n, xcd = blockIdx.x % 8, rem = total % 8;
+  const int K = p.K, T = p.T;
+  const int total = p.tiles_m * p.tiles_n, xcd = blockIdx.x % 8, rem = total % 8;
   const int id = xcd * (total / 8) + min(xcd, rem) + (int)blockIdx.x / 8;
-  const int gi = id / (group_m * tiles_n), in = id - gi * (group_m * tiles_n);
-  const int gm = min(group_m, tiles_m - gi * group_m);
-  const int m0 = (gi * group_m + in % gm) * BM, n0 = (in / gm) * BN;
+  const int gi = id / (p.group_m * p.tiles_n), in = id - gi * (p.group_m * p.tiles_n);
+  const int gm = min(p.group_m, p.tiles_m - gi * p.group_m);
+  const int tm = gi * p.group_m + in % gm, n0 = (in / gm) * BN;
+  const int mat = PAIR || tm < p.tend[0] ? 0 : tm < p.tend[1] ? 1 : 2;
+  const int M = mat == 0 ? p.rows[0] : mat == 1 ? p.rows[1] : p.rows[2];
+  const float* const w = mat == 0 ? p.w[0] : mat == 1 ? p.w[1] : p.w[2];
+  float* const y = mat == 0 ? p.y[0] : mat == 1 ? p.y[1] : p.y[2];
+  const float* const x = p.x;
+  const int m0 = PAIR ? tm * (BM / 2) : (tm - (mat == 0 ? 0 : mat == 1 ? p.tend[0] : p.tend[1])) * BM;
 
   float* stage = lds + wave * STAGE;
   const int lrow = lane / C16, lp = lane % C16;
   // This lane's first column; the last lanes move back so that their WN
   // columns stay inside the row (and store only their own).
   const int nom = n0 + WN * ln, col0 = min(nom, T - WN);
-  const float* wt = w + (size_t)m0 * K;
+  const float* const wt = w + (size_t)m0 * K;
+  [[maybe_unused]] const float* const wt2 = PAIR ? p.w[1] + (size_t)m0 * K : nullptr;
   const int mlast = M - 1 - m0;  // rows past it read row mlast and store nothing
+  // Tile row r: its matrix and its row there behind m0.
+  auto wbase = [&](int r) { return PAIR && (r & 16) ? wt2 : wt; };
+  auto wrow = [&](int r) { return min(PAIR ? 16 * (r >> 5) + (r & 15) : r, mlast); };
   uint32_t woff[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int r = RPL * i + lrow;
-    woff[i] = (uint32_t)min(r, mlast) * (uint32_t)K + 4u * (uint32_t)(lp ^ (r & (C16 - 1)));
+    woff[i] = (uint32_t)wrow(r) * (uint32_t)K + 4u * (uint32_t)(lp ^ (r & (C16 - 1)));
   }
   const uint32_t xoff = (uint32_t)(8 * hh) * (uint32_t)T + (uint32_t)col0;
   const int nfull = K / CK;
@@ -269,9 +310,10 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(const float* __re
     [[maybe_unused]] float sa[WM], sb[WN];
     auto load_w = [&](int c) {
       const float* src = wt + (size_t)c * CK;
+      [[maybe_unused]] const float* src2 = PAIR ? wt2 + (size_t)c * CK : nullptr;
 #pragma unroll
-      for (int i = 0; i < NL; ++i) {
-        const FVec<4>::T t = *(const FVec<4>::T*)(src + woff[i]);
+      for (int i = 0; i < NL; ++i) {  // RPL divides 16: one matrix per load
+        const FVec<4>::T t = *(const FVec<4>::T*)((PAIR && (RPL * i & 16) ? src2 : src) + woff[i]);
         wr[i] = f32x4{t[0], t[1], t[2], t[3]};
       }
     };
@@ -319,7 +361,7 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(const float* __re
           for (int k = c * CK + hh; k < min(c * CK + CK, K); k += 2) {
 #pragma unroll
             for (int a = 0; a < WM; ++a)
-              ma[a] = fmaxf(ma[a], fabsf(wt[(size_t)min(32 * a + ln, mlast) * K + k]));
+              ma[a] = fmaxf(ma[a], fabsf(wbase(ln)[(size_t)wrow(32 * a + ln) * K + k]));
 #pragma unroll
             for (int b = 0; b < WN; ++b) mb[b] = fmaxf(mb[b], fabsf(x[(size_t)k * T + col0 + b]));
           }
@@ -338,31 +380,82 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(const float* __re
       wave_lds_sync();
       return __any(bad);
     };
+    auto split_b = [&](const float (*xv)[WN], int b) {
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = xv[j][b];
+      return split8(v, sb[b]);
+    };
+    // MFMA i of the 3 WM of a column block: lo hi', hi lo', hi hi'.
+    auto product = [&](const Split8* A, const Split8& B, int b, int i) {
+      const int a = i % WM;
+      acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(i < WM ? A[a].lo : A[a].hi),
+                                                         as_f16(i / WM == 1 ? B.lo : B.hi), acc[a][b], 0, 0, 0);
+    };
+    // Step s on operands split before (A, B of column block 0); splits those
+    // of the next step (its x in xn, its A if next_a) and of the other column
+    // blocks between the MFMAs.  load_next overwrites xv once it is split.
+    auto piped = [&](int s, const float (*xv)[WN], const float (*xn)[WN], Split8* A, Split8& B, bool next_a,
+                     auto load_next) {
+      constexpr int N = 3 * WM;
+      float va[WM][8];
+      Split8 A2[WM];
+      if (next_a)
+#pragma unroll
+        for (int a = 0; a < WM; ++a) read_a(a, s + 1, va[a]);
+#pragma unroll
+      for (int b = 0; b < WN; ++b) {
+        Split8 B2;
+        const int nb = (b + 1) % WN;
+        if (b == WN - 1) {
+          __builtin_amdgcn_sched_barrier(0);
+          load_next();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          product(A, B, b, i);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 4 * i / N; j < 4 * (i + 1) / N; ++j) {  // of the next column block
+            const float(*src)[WN] = nb ? xv : xn;
+            uint32_t h, l;
+            split2(src[2 * j][nb], src[2 * j + 1][nb], sb[nb], h, l);
+            B2.hi[j] = h;
+            B2.lo[j] = l;
+          }
+          const int at = b * N + i;
+          if (next_a)
+#pragma unroll
+            for (int u = 4 * WM * at / (N * WN); u < 4 * WM * (at + 1) / (N * WN); ++u) {  // of the next step's A
+              const int a = u / 4, j = u % 4;
+              uint32_t h, l;
+              split2(va[a][2 * j], va[a][2 * j + 1], sa[a], h, l);
+              A2[a].hi[j] = h;
+              A2[a].lo[j] = l;
+            }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        B = B2;
+      }
+      if (next_a)
+#pragma unroll
+        for (int a = 0; a < WM; ++a) A[a] = A2[a];
+    };
     auto step = [&](int s, const float (*xv)[WN]) {
       if constexpr (SPLIT) {
-        f16x8 ah[WM], al[WM];
+        Split8 A[WM];
 #pragma unroll
         for (int a = 0; a < WM; ++a) {
           float v[8];
           read_a(a, s, v);
-          split8(v, sa[a], ah[a], al[a]);
+          A[a] = split8(v, sa[a]);
         }
 #pragma unroll
         for (int b = 0; b < WN; ++b) {
-          float v[8];
+          const Split8 B = split_b(xv, b);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) v[j] = xv[j][b];
-          f16x8 bh, bl;
-          split8(v, sb[b], bh, bl);
-#pragma unroll
-          for (int a = 0; a < WM; ++a)
-            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[a], bh, acc[a][b], 0, 0, 0);
-#pragma unroll
-          for (int a = 0; a < WM; ++a)
-            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[a], bl, acc[a][b], 0, 0, 0);
-#pragma unroll
-          for (int a = 0; a < WM; ++a)
-            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[a], bh, acc[a][b], 0, 0, 0);
+          for (int i = 0; i < 3 * WM; ++i) product(A, B, b, i);
         }
       } else {
         // MFMA j pairs k 8 hh + j of the two lane halves
@@ -386,6 +479,7 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(const float* __re
       load_w(wave);
 #pragma unroll
       for (int s = 0; s < XD; ++s) load_x(wave * CK + 16 * s, xr[s]);
+      [[maybe_unused]] Split8 A[WM], B;
       for (int n = 0, c = wave; n < nmine; ++n, c += KW) {
         put_w();
         const int cn = min(c + KW, nfull - 1);
@@ -395,12 +489,27 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(const float* __re
         if (SPLIT && n == 0) {
           if (scales(xr[0])) return true;
           scaled = true;
+          if constexpr (SPLIT) B = split_b(xr[0], 0);
         }
+        if constexpr (SPLIT)
+#pragma unroll
+          for (int a = 0; a < WM; ++a) {
+            float v[8];
+            read_a(a, 0, v);
+            A[a] = split8(v, sa[a]);
+          }
 #pragma unroll
         for (int s = 0; s < ST; ++s) {
-          step(s, xr[s % XD]);
-          __builtin_amdgcn_sched_barrier(0);
-          load_x(s + XD < ST ? c * CK + 16 * (s + XD) : cn * CK + 16 * (s + XD - ST), xr[s % XD]);
+          auto load_next = [&]() {
+            load_x(s + XD < ST ? c * CK + 16 * (s + XD) : cn * CK + 16 * (s + XD - ST), xr[s % XD]);
+          };
+          if constexpr (SPLIT) {
+            piped(s, xr[s % XD], xr[(s + 1) % XD], A, B, s + 1 < ST, load_next);
+          } else {
+            step(s, xr[s % XD]);
+            __builtin_amdgcn_sched_barrier(0);
+            load_next();
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -410,7 +519,7 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(const float* __re
 #pragma unroll
       for (int i = 0; i < NL; ++i) {
         const int r = RPL * i + lrow, kk = k0 + 4 * (lp ^ (r & (C16 - 1)));
-        const float* src = wt + (size_t)min(r, mlast) * K;
+        const float* src = wbase(RPL * i) + (size_t)wrow(r) * K;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float v = src[min(kk + e, K - 1)];
@@ -458,8 +567,10 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(const float* __re
   // wave could not split) nothing is stored and the result is false.
   auto finish = [&](auto check_tag, bool bad) -> bool {
     constexpr bool CHECK = decltype(check_tag)::value;
-    constexpr int UPT = (WM * 4 + KW - 1) / KW;  // (a, q) units per wave
-    __syncthreads();                             // the staging areas are free
+    // Units of four rows per lane: (a, q) of the tile, for PAIR q = 0, 1 (gate)
+    // with q + 2 (up).
+    constexpr int QN = PAIR ? 2 : 4, UPT = (WM * QN + KW - 1) / KW;  // units per wave
+    __syncthreads();                                                 // the staging areas are free
     f32x4* part = (f32x4*)lds + wave * (PART / 4);
 #pragma unroll
     for (int a = 0; a < WM; ++a)
@@ -472,39 +583,51 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(const float* __re
     __syncthreads();
     f32x4 sum[UPT][WN];
     float z = 0.f;
+    auto added = [&](int a, int b, int q) {
+      const f32x4* src = (const f32x4*)lds + ((a * WN + b) * 4 + q) * 64 + lane;
+      f32x4 t = src[0];
+#pragma unroll
+      for (int k = 1; k < KW; ++k) t += src[k * (PART / 4)];
+      if (CHECK) z += t.x * 0.f + t.y * 0.f + (t.z * 0.f + t.w * 0.f);
+      return t;
+    };
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
       const int aq = wave + KW * u;
-      if (aq >= WM * 4) break;
-      const f32x4* src = (const f32x4*)lds + ((aq >> 2) * WN * 4 + (aq & 3)) * 64 + lane;
+      if (aq >= WM * QN) break;
 #pragma unroll
       for (int b = 0; b < WN; ++b) {
-        f32x4 t = src[b * 256];
+        f32x4 t = added(aq / QN, b, aq % QN);
+        if constexpr (PAIR) {
+          const f32x4 up = added(aq / QN, b, aq % QN + 2);
 #pragma unroll
-        for (int k = 1; k < KW; ++k) t += src[b * 256 + k * (PART / 4)];
+          for (int e = 0; e < 4; ++e) t[e] = t[e] * (1.0f / (1.0f + expf(-t[e]))) * up[e];  // gpuSiluMul
+        }
         sum[u][b] = t;
-        if (CHECK) z += t.x * 0.f + t.y * 0.f + (t.z * 0.f + t.w * 0.f);
       }
     }
     if (CHECK && __syncthreads_or(bad || z != 0.f)) return false;
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
       const int aq = wave + KW * u;
-      if (aq >= WM * 4) break;
+      if (aq >= WM * QN) break;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int m = m0 + 32 * (aq >> 2) + 8 * (aq & 3) + 4 * hh + e;
+        const int m = m0 + (PAIR ? 16 : 32) * (aq / QN) + 8 * (aq % QN) + 4 * hh + e;
         if (m >= M || nom >= T) continue;
-        float* dst = y + (size_t)m * T + col0;
+        const size_t at = (size_t)m * T + col0;
+        float* dst = y + at;
         if (WN > 1 && col0 == nom) {
-          typename FVec<WN == 1 ? 2 : WN>::T v;
+          typedef typename FVec<WN == 1 ? 2 : WN>::T V;
+          V v = {};
+          if (p.res) v = *(const V*)(p.res + at);
 #pragma unroll
-          for (int b = 0; b < WN; ++b) v[b] = sum[u][b][e];
-          *(typename FVec<WN == 1 ? 2 : WN>::T*)dst = v;
+          for (int b = 0; b < WN; ++b) v[b] = p.res ? v[b] + sum[u][b][e] : sum[u][b][e];
+          *(V*)dst = v;
         } else {
 #pragma unroll
           for (int b = 0; b < WN; ++b)
-            if (col0 + b >= nom) dst[b] = sum[u][b][e];
+            if (col0 + b >= nom) dst[b] = p.res ? p.res[at + b] + sum[u][b][e] : sum[u][b][e];
         }
       }
     }
@@ -537,59 +660,77 @@ constexpr SplitVariant kSplit[] = {
     {64, 128, 1, 5.57f, 11.78f, 11.37f}, // 4 waves
 };
 
-LinearPlan linear_plan(int M, int K, int T, const float* w, const float* x) {
+LinearPlan linear_plan(const LinearCall& c) {
   LinearPlan p{};
-  if (T == 1) {
-    p.gemv = true;
-    p.vec = (K % 4 == 0) && aligned16(w) && aligned16(x);
-    p.wpr = M >= 2048 ? 1 : 4;
-    p.grid_x = (M + 4 / p.wpr - 1) / (4 / p.wpr);
-    return p;
-  }
   float best = 0.f;
   const int cus = cu_count();
   for (int v = 0; v < (int)(sizeof(kSplit) / sizeof(kSplit[0])); ++v) {
     const SplitVariant& s = kSplit[v];
-    if (T < s.bn / 32) continue;  // a lane holds bn / 32 columns
-    const long long tm = ((long long)M + s.bm - 1) / s.bm, tn = ((long long)T + s.bn - 1) / s.bn;
-    const long long rounds = (tm * tn + (long long)cus * s.per_cu - 1) / ((long long)cus * s.per_cu);
-    const float t = 2.f + (float)rounds * (s.fixed + (rounds > 1 ? s.more : s.one) * (float)K * 1e-3f);
+    if (c.T < s.bn / 32) continue;  // a lane holds bn / 32 columns
+    const int bm = c.pair ? s.bm / 2 : s.bm;
+    long long tm[3] = {0, 0, 0};
+    for (int i = 0; i < (c.pair ? 1 : c.nmat); ++i) tm[i] = ((long long)c.rows[i] + bm - 1) / bm;
+    const long long all = tm[0] + tm[1] + tm[2], tn = ((long long)c.T + s.bn - 1) / s.bn;
+    if (all * tn > 0x7FFFFFFFLL) continue;
+    const long long rounds = (all * tn + (long long)cus * s.per_cu - 1) / ((long long)cus * s.per_cu);
+    const float t = 2.f + (float)rounds * (s.fixed + (rounds > 1 ? s.more : s.one) * (float)c.K * 1e-3f);
     if (p.tiles_m == 0 || t < best) {
       best = t;
       p.variant = v;
-      p.tiles_m = (int)tm;
+      p.tiles_m = (int)all;
       p.tiles_n = (int)tn;
+      p.tend[0] = (int)tm[0];
+      p.tend[1] = (int)(tm[0] + tm[1]);
     }
   }
   return p;
 }
 
 template <int WM, int WN, int KW, int CK, int XD>
-static void launch_split(float* y, const float* x, const float* w, int K, int M, int T, const LinearPlan& p,
-                         hipStream_t stream) {
-  hipLaunchKernelGGL((linear_split_kernel<WM, WN, KW, CK, XD>), dim3((unsigned)p.tiles_m * (unsigned)p.tiles_n),
-                     dim3(64 * KW), 0, stream, w, x, y, M, K, T, p.tiles_m, p.tiles_n, WN == 4 ? 4 : 8);
+static void launch_split(const SplitArgs& a, bool pair, hipStream_t stream) {
+  const dim3 grid((unsigned)a.tiles_m * (unsigned)a.tiles_n), block(64 * KW);
+  if (pair) hipLaunchKernelGGL((linear_split_kernel<WM, WN, KW, CK, XD, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((linear_split_kernel<WM, WN, KW, CK, XD, false>), grid, block, 0, stream, a);
+}
+
+hipError_t linear_cols_launch(const LinearCall& c, hipStream_t stream) {
+  const LinearPlan p = linear_plan(c);
+  if (p.tiles_m == 0) return hipErrorInvalidValue;
+  SplitArgs a{};
+  for (int i = 0; i < c.nmat; ++i) {
+    a.w[i] = c.w[i];
+    a.y[i] = c.y[i];
+    a.rows[i] = c.rows[i];
+  }
+  a.tend[0] = p.tend[0];
+  a.tend[1] = p.tend[1];
+  a.x = c.x;
+  a.res = c.res;
+  a.K = c.K;
+  a.T = c.T;
+  a.tiles_m = p.tiles_m;
+  a.tiles_n = p.tiles_n;
+  a.group_m = kSplit[p.variant].bn == 128 ? 4 : 8;
+  if (p.variant == 0) launch_split<1, 1, 8, 64, 4>(a, c.pair, stream);
+  else if (p.variant == 1) launch_split<2, 2, 8, 32, 2>(a, c.pair, stream);
+  else if (p.variant == 2) launch_split<2, 2, 4, 32, 2>(a, c.pair, stream);
+  else launch_split<2, 4, 4, 64, 2>(a, c.pair, stream);
+  return hipGetLastError();
 }
 
 hipError_t linear_col_launch(float* y, const float* x, const float* w, int K, int M, int T,
                              hipStream_t stream) {
-  const LinearPlan p = linear_plan(M, K, T, w, x);
-  if (p.gemv) {
-    const dim3 grid(p.grid_x), block(256);
-    if (p.wpr == 1) {
-      if (p.vec) hipLaunchKernelGGL((linear_gemv_kernel<1, true>), grid, block, 0, stream, w, x, y, M, K);
-      else hipLaunchKernelGGL((linear_gemv_kernel<1, false>), grid, block, 0, stream, w, x, y, M, K);
-    } else {
-      if (p.vec) hipLaunchKernelGGL((linear_gemv_kernel<4, true>), grid, block, 0, stream, w, x, y, M, K);
-      else hipLaunchKernelGGL((linear_gemv_kernel<4, false>), grid, block, 0, stream, w, x, y, M, K);
-    }
-    return hipGetLastError();
+  if (T > 1) return linear_cols_launch(LinearCall{1, {w}, {y}, {M}, x, nullptr, false, K, T}, stream);
+  const bool vec = K % 4 == 0 && aligned16(w) && aligned16(x);
+  const int wpr = M >= 2048 ? 1 : 4;
+  const dim3 grid((M + 4 / wpr - 1) / (4 / wpr)), block(256);
+  if (wpr == 1) {
+    if (vec) hipLaunchKernelGGL((linear_gemv_kernel<1, true>), grid, block, 0, stream, w, x, y, M, K);
+    else hipLaunchKernelGGL((linear_gemv_kernel<1, false>), grid, block, 0, stream, w, x, y, M, K);
+  } else {
+    if (vec) hipLaunchKernelGGL((linear_gemv_kernel<4, true>), grid, block, 0, stream, w, x, y, M, K);
+    else hipLaunchKernelGGL((linear_gemv_kernel<4, false>), grid, block, 0, stream, w, x, y, M, K);
   }
-  if ((long long)p.tiles_m * p.tiles_n > 0x7FFFFFFFLL) return hipErrorInvalidValue;
-  if (p.variant == 0) launch_split<1, 1, 8, 64, 4>(y, x, w, K, M, T, p, stream);
-  else if (p.variant == 1) launch_split<2, 2, 8, 32, 2>(y, x, w, K, M, T, p, stream);
-  else if (p.variant == 2) launch_split<2, 2, 4, 32, 2>(y, x, w, K, M, T, p, stream);
-  else launch_split<2, 4, 4, 64, 2>(y, x, w, K, M, T, p, stream);
   return hipGetLastError();
 }
 

@@ -542,6 +542,18 @@ static int check_workspace(const hl_forward_scratch* s, size_t need) {
   return HL_OK;
 }
 
+// One launch of the fp32 projections that share x (LinearCall); a single
+// column goes through the GEMVs, a residual (onto y[0] itself) by way of tmp.
+static int prefill_linear(const LinearCall& c, void* stream, float* tmp = nullptr) {
+  if (c.T > 1) {
+    const hipError_t e = linear_cols_launch(c, (hipStream_t)stream);
+    return e == hipSuccess ? HL_OK : set_error(HL_EHIP, "prefill linear launch: %s", hipGetErrorString(e));
+  }
+  for (int i = 0; i < c.nmat; ++i)
+    HL_TRY(hl_gpu_linear_col(c.res ? tmp : c.y[i], c.x, c.w[i], c.K, c.rows[i], 1, stream));
+  return c.res ? hl_gpu_add(c.y[0], c.res, tmp, c.rows[0], stream) : HL_OK;
+}
+
 int hl_forward_prefill(const hl_model_desc* m, hl_kv_cache_desc* c, const hl_forward_scratch* s,
                        const int32_t* tokens_dev, int T, float* logits, void* stream) {
   HL_TRY(check_model(m, true));
@@ -570,22 +582,23 @@ int hl_forward_prefill(const hl_model_desc* m, hl_kv_cache_desc* c, const hl_for
   for (int l = 0; l < m->n_layer; ++l) {
     const hl_layer_desc& L = m->layers[l];
     HL_TRY(hl_gpu_rmsnorm_cols(xn, x, L.attn_norm, E, T, eps, stream));
-    HL_TRY(hl_gpu_linear_col(t0, xn, (const float*)L.wq, E, qdim, T, stream));
-    HL_TRY(hl_gpu_linear_col(t1, xn, (const float*)L.wk, E, kvdim, T, stream));
-    HL_TRY(hl_gpu_linear_col(t2, xn, (const float*)L.wv, E, kvdim, T, stream));
+    const float *wq = (const float*)L.wq, *wk = (const float*)L.wk, *wv = (const float*)L.wv;
+    HL_TRY(prefill_linear({3, {wq, wk, wv}, {t0, t1, t2}, {qdim, kvdim, kvdim}, xn, nullptr, false, E, T}, stream));
     // qk-norm, RoPE at positions 0 .. T-1, the cache write of columns
     // 0 .. T-1 and causal attention (naive.nim:4066-4078) in one call
     hl_prefill_args p;
     prefill_args(p, m, c, l, t0, t1, t2, xn, T);
     HL_TRY(hl_attn_prefill(&p, pws, pws_bytes, stream));
-    HL_TRY(hl_gpu_linear_col(t0, xn, (const float*)L.wo, qdim, E, T, stream));
-    HL_TRY(hl_gpu_add(x, x, t0, E * T, stream));
+    HL_TRY(prefill_linear({1, {(const float*)L.wo}, {x}, {E}, xn, x, false, qdim, T}, stream, t0));
     HL_TRY(hl_gpu_rmsnorm_cols(xn, x, L.ffn_norm, E, T, eps, stream));
-    HL_TRY(hl_gpu_linear_col(t0, xn, (const float*)L.w_gate, E, m->n_ff, T, stream));
-    HL_TRY(hl_gpu_linear_col(t1, xn, (const float*)L.w_up, E, m->n_ff, T, stream));
-    HL_TRY(hl_gpu_silu_mul(t2, t0, t1, m->n_ff * T, stream));
-    HL_TRY(hl_gpu_linear_col(t0, t2, (const float*)L.w_down, m->n_ff, E, T, stream));
-    HL_TRY(hl_gpu_add(x, x, t0, E * T, stream));
+    const float *wg = (const float*)L.w_gate, *wu = (const float*)L.w_up;
+    if (T > 1) {
+      HL_TRY(prefill_linear({2, {wg, wu}, {t2}, {m->n_ff, m->n_ff}, xn, nullptr, true, E, T}, stream));
+    } else {
+      HL_TRY(prefill_linear({2, {wg, wu}, {t0, t1}, {m->n_ff, m->n_ff}, xn, nullptr, false, E, T}, stream));
+      HL_TRY(hl_gpu_silu_mul(t2, t0, t1, m->n_ff, stream));
+    }
+    HL_TRY(prefill_linear({1, {(const float*)L.w_down}, {x}, {E}, t2, x, false, m->n_ff, T}, stream, t0));
   }
   HL_TRY(hl_gpu_rmsnorm_cols(xn, x, m->output_norm, E, T, eps, stream));
   HL_TRY(hl_gpu_linear_col(logits, xn, (const float*)m->output, E, m->n_vocab, T, stream));

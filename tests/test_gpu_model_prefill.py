@@ -206,3 +206,67 @@ def test_decode_timed_matches_decode(hl, orc):
     with pytest.raises(_lib.HLError, match="capture"):
         with torch.cuda.graph(g, stream=s):
             twins[1].decode_timed(stream=s)
+
+
+# The merged prefill launches (Q/K/V as one row list, gate/up with SiLU * up
+# on the sums, the residual added on the way out) at ragged rows of each
+# matrix and every tile size of either, against float64.  wide: gate and up
+# rows with one element far above the rest, whose tiles leave the split's
+# range and are computed a second time (w_down takes the size out again).
+# Bound: the fp32 model bar, on logits and on the cached K and V.
+@pytest.mark.parametrize("E,H,Hkv,ff,T,wide", [(72, 2, 1, 100, 3, False), (160, 4, 2, 331, 37, True),
+                                               (512, 8, 2, 1003, 301, True), (512, 16, 4, 4003, 301, False),
+                                               (512, 8, 2, 4003, 1000, True), (256, 32, 16, 2057, 303, False),
+                                               (1024, 16, 4, 2500, 300, True)])
+def test_prefill_merged_launches(hl, E, H, Hkv, ff, T, wide):
+    from hippo_leap_amd.model import DenseModel
+    print(f"prefill merged launches E={E} H={H}/{Hkv} ff={ff} T={T} wide={wide}", flush=True)
+    D, V = 64, 70
+    cfg = dict(n_layer=2, n_emb=E, n_head=H, n_head_kv=Hkv, head_dim=D, rope_dim=D, n_ff=ff, n_vocab=V,
+               max_len=T + 5, rms_eps=1e-6, rope_base=1e4)
+    g = torch.Generator(device="cuda").manual_seed(E + ff + T)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    shapes = {"wq": (H * D, E), "wk": (Hkv * D, E), "wv": (Hkv * D, E), "wo": (E, H * D), "w_gate": (ff, E),
+              "w_up": (ff, E), "w_down": (E, ff)}
+    layers = []
+    for _ in range(2):
+        L = {n: rnd(*s) / s[1] ** 0.5 for n, s in shapes.items()}
+        if wide:
+            for n, r in (("w_up", 7), ("w_gate", ff - 1)):
+                L[n][r, -1] += 3e5
+                L["w_down"][:, r] *= 3e-6
+        L["attn_norm"], L["ffn_norm"] = 1 + 0.1 * rnd(E), 1 + 0.1 * rnd(E)
+        L["k_cache"], L["v_cache"] = (torch.zeros(Hkv * D, T + 5, device="cuda") for _ in range(2))
+        layers.append(L)
+    emb, onorm, out = rnd(V, E), 1 + 0.1 * rnd(E), rnd(V, E) / E ** 0.5
+    m = DenseModel(torch, cfg, emb, onorm, out, 0, layers, max_tokens=T)
+    tokens = torch.randint(V, (T,), device="cuda", generator=g, dtype=torch.int32)
+    logits = m.prefill(tokens)
+    torch.cuda.synchronize()
+
+    norm = lambda x, w: x / (x.pow(2).mean(0, True) + 1e-6).sqrt() * w.double()[:, None]
+    ang = torch.arange(T, device="cuda").double() * (1e4 ** (-torch.arange(D // 2, device="cuda").double() * 2 / D))[:, None]
+    c, s = ang.cos(), ang.sin()
+
+    def rope(x):
+        a, b = x.view(-1, D, T).split(D // 2, 1)
+        return torch.cat([a * c - b * s, a * s + b * c], 1)
+
+    x = emb.double()[tokens.long()].T
+    for i, L in enumerate(layers):
+        w = {n: L[n].double() for n in shapes}
+        xn = norm(x, L["attn_norm"])
+        q, k, v = rope(w["wq"] @ xn), rope(w["wk"] @ xn), (w["wv"] @ xn).view(-1, D, T)
+        for cache, ref in ((m.cache.k[i], k), (m.cache.v[i], v)):
+            got = cache.view(torch.float32).view(Hkv * D, T + 5)[:, :T]
+            assert rel_err(got.cpu(), ref.reshape(Hkv * D, T).cpu()) < TOL_F32
+        heads = []
+        for h in range(H):
+            p = (q[h].T @ k[h * Hkv // H] / D ** 0.5).masked_fill(
+                torch.ones(T, T, device="cuda", dtype=torch.bool).triu(1), float("-inf")).softmax(1)
+            heads.append(v[h * Hkv // H] @ p.T)
+        x = x + w["wo"] @ torch.cat(heads)
+        xn = norm(x, L["ffn_norm"])
+        x = x + w["w_down"] @ (torch.nn.functional.silu(w["w_gate"] @ xn) * (w["w_up"] @ xn))
+    ref = out.double() @ norm(x, onorm)
+    assert rel_err(logits.cpu(), ref.cpu()) < TOL_F32
