@@ -134,8 +134,9 @@ __device__ __forceinline__ bool arrive_last(unsigned int* slot, int S) {
 struct NoTail {
   __device__ void operator()() const {}
 };
-template <int D, typename Tail = NoTail>
-__device__ void finish_workgroup(const DecodeParams& p, const float* sm_m, const float* sm_l,
+// WIDE: num_splits > 8.
+template <int D, bool WIDE, typename Tail = NoTail>
+__device__ void finish_workgroup(const DecodeParams& p, float* sm_m, const float* sm_l,
                                  const float* sm_o, int hc, int b, int kvh, int chunk, int hq0,
                                  int split, int hstride, Tail after = Tail()) {
   const int tid = threadIdx.x;
@@ -176,35 +177,36 @@ __device__ void finish_workgroup(const DecodeParams& p, const float* sm_m, const
   after();
   if (!last) return;
 
-  // Fold all splits, 8 at a time: each chunk's m, l and o loads are issued
-  // together (one memory round trip per 8 splits), then merged into a
-  // running (max, sum, accumulator) per output element.
-  for (int idx = tid; idx < hc * D; idx += 256) {
+  // Folds splits from .. to - 1 of one output element into (max, sum,
+  // accumulator), U at a time: a batch's m, l and o loads are issued together
+  // (one memory round trip).
+  auto fold = [&](auto ucount, int idx, int from, int to, float& M, float& lsum, float& osum) {
+    constexpr int U = decltype(ucount)::value;
     const int h = idx / D, d = idx % D;
     const long long row = (long long)b * p.n_head + hq0 + h;
     const float* ml = p.ws_ml + row * S * 2;
     const float* wo = p.ws_o + row * S * D + d;
-    float M = -INFINITY, lsum = 0.f, osum = 0.f;
-    for (int s0 = 0; s0 < S; s0 += 8) {
-      float m[8], l[8], x[8];
+    M = -INFINITY, lsum = 0.f, osum = 0.f;
+    for (int s0 = from; s0 < to; s0 += U) {
+      float m[U], l[U], x[U];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int sp = min(s0 + u, S - 1);
+      for (int u = 0; u < U; ++u) {
+        const int sp = min(s0 + u, to - 1);
         m[u] = load_agent(&ml[2 * sp]);
         l[u] = load_agent(&ml[2 * sp + 1]);
         x[u] = load_agent(&wo[(long long)sp * D]);
       }
       float mc = M;
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (s0 + u < S) mc = fmaxf(mc, m[u]);
+      for (int u = 0; u < U; ++u)
+        if (s0 + u < to) mc = fmaxf(mc, m[u]);
       if (mc == -INFINITY) continue;  // no columns so far (empty splits)
       const float r = fast_exp2(M - mc);
       lsum *= r;
       osum *= r;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        if (s0 + u < S) {
+      for (int u = 0; u < U; ++u) {
+        if (s0 + u < to) {
           const float w = fast_exp2(m[u] - mc);
           lsum += w * l[u];
           osum += w * x[u];
@@ -212,7 +214,51 @@ __device__ void finish_workgroup(const DecodeParams& p, const float* sm_m, const
       }
       M = mc;
     }
-    p.out[row * D + d] = osum / lsum;
+  };
+  const long long out0 = ((long long)b * p.n_head + hq0) * D;
+  float M, lsum, osum;
+  if constexpr (!WIDE) {
+    for (int idx = tid; idx < hc * D; idx += 256) {
+      fold(std::integral_constant<int, 8>{}, idx, 0, S, M, lsum, osum);
+      p.out[out0 + idx] = osum / lsum;
+    }
+  } else {
+    // The round trips are what the fold costs: 16 splits a trip, and with
+    // fewer output elements than threads, groups of threads fold a share of
+    // the splits each and meet in LDS (the waves' states there are dead).
+    // One sequence, 32 heads over 8, D = 128, 2000 columns: 14.4 -> 13.9 us
+    // (8 a trip before); over 4 heads, 4000 columns: 21.8 -> 19.5; D = 64,
+    // 8000: 16.6 -> 15.7; fp32, D = 128, 2000: 19.7 -> 18.8.
+    const int items = hc * D;
+    const int groups = items <= 128 ? min(256 / items, (S + 15) / 16) : 1;
+    const int share = (S + groups - 1) / groups;
+    if (groups == 1) {
+      for (int idx = tid; idx < items; idx += 256) {
+        fold(std::integral_constant<int, 16>{}, idx, 0, S, M, lsum, osum);
+        p.out[out0 + idx] = osum / lsum;
+      }
+    } else {
+      float* meet = sm_m;  // [groups][items][3], at most 256 x 3
+      const int grp = tid / items, idx = tid - grp * items;
+      if (grp < groups) {
+        fold(std::integral_constant<int, 16>{}, idx, min(grp * share, S), min(grp * share + share, S), M, lsum, osum);
+        meet[3 * tid] = M;
+        meet[3 * tid + 1] = lsum;
+        meet[3 * tid + 2] = osum;
+      }
+      __syncthreads();
+      if (tid < items) {
+        for (int i = 1; i < groups; ++i) M = fmaxf(M, meet[3 * (i * items + tid)]);
+        lsum = osum = 0.f;
+        for (int i = 0; i < groups; ++i) {
+          const float* q = meet + 3 * (i * items + tid);
+          const float w = q[0] == -INFINITY ? 0.f : fast_exp2(q[0] - M);
+          lsum += w * q[1];
+          osum += w * q[2];
+        }
+        p.out[out0 + tid] = osum / lsum;
+      }
+    }
   }
   HL_STAMP(5);
   if (tid == 0) __hip_atomic_store(slot, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -227,7 +273,7 @@ __device__ void finish_workgroup(const DecodeParams& p, const float* sm_m, const
 // past the chunk's heads score a zero q row and are never written out; every
 // slot is computed without a branch, so the heads' dependency chains (dot
 // products, wave reductions) interleave instead of running one after another.
-template <int D, bool V4, int HC>
+template <int D, bool V4, int HC, bool WIDE>
 __global__ __launch_bounds__(256) void decode_f32_kernel(DecodeParams p) {
   // D = 128 keeps one head at a time (uniform branches): interleaving every
   // head's chains there needs more registers than the kernel has.
@@ -414,7 +460,7 @@ __global__ __launch_bounds__(256) void decode_f32_kernel(DecodeParams p) {
   }
   __syncthreads();
   HL_STAMP(3);
-  finish_workgroup<D>(p, sm_m, sm_l, sm_o, hc, b, kvh, chunk, hq0, split, HC);
+  finish_workgroup<D, WIDE>(p, sm_m, sm_l, sm_o, hc, b, kvh, chunk, hq0, split, HC);
 }
 
 // ---------------------------------------------------------------------------
@@ -499,7 +545,7 @@ __device__ __forceinline__ u16x8 mask_row8(u16x8 r, int col, int lim) {
 // tighter bounds that spilled: the fused step at head dim 128 (Llama-3-8B-
 // shaped layer, one sequence, 2K columns) 15.3 -> 13.0 us; the scalar-load
 // kernel at head dim 64 (c3 shape with an odd cache length) 40.5 -> 28.8 us.
-template <int D, int DT, bool VEC, bool PIPE, bool STEP, bool PG = false>
+template <int D, int DT, bool VEC, bool PIPE, bool STEP, bool PG, bool WIDE>
 __global__ __launch_bounds__(256, PIPE ? (D == 64 ? 2 : 1) : (D == 64 ? (VEC ? 4 : 2) : (STEP ? 1 : 2))) void decode_mfma_kernel(DecodeParams p) {
   static_assert(!PG || VEC, "paged caches are read with vector loads only");
   // MFMA operand type: the storage type, except fp8 caches, which are
@@ -941,7 +987,7 @@ __global__ __launch_bounds__(256, PIPE ? (D == 64 ? 2 : 1) : (D == 64 ? (VEC ? 4
     // end of the kernel to write back (c3 step: 12.78 -> 12.64 us; issued
     // before the tiles instead, the plain stores cost as much, because the
     // tile waits count them).
-    finish_workgroup<D>(p, sm_m, sm_l, sm_o, hc, b, kvh, chunk, hq0, split, HS, [&]() {
+    finish_workgroup<D, WIDE>(p, sm_m, sm_l, sm_o, hc, b, kvh, chunk, hq0, split, HS, [&]() {
       if (has_new && chunk == 0) {
         for (int i = tid; i < 2 * D; i += 256) {
           const int dd = i < D ? i : i - D;
@@ -956,7 +1002,7 @@ __global__ __launch_bounds__(256, PIPE ? (D == 64 ? 2 : 1) : (D == 64 ? (VEC ? 4
       }
     });
   } else {
-    finish_workgroup<D>(p, sm_m, sm_l, sm_o, hc, b, kvh, chunk, hq0, split, HS);
+    finish_workgroup<D, WIDE>(p, sm_m, sm_l, sm_o, hc, b, kvh, chunk, hq0, split, HS);
   }
 }
 
@@ -1006,39 +1052,48 @@ typedef void (*KernelFn)(DecodeParams);
 
 // The prefetching kernel exists for the 16-byte path only (the element-wise
 // loads of unaligned caches would not fit its registers).
-template <int D, bool V4>
+template <int D, bool V4, bool W>
 KernelFn pick_f32_hc(int hc) {
-  if (hc <= 1) return decode_f32_kernel<D, V4, 1>;
-  if (hc <= 2) return decode_f32_kernel<D, V4, 2>;
-  return hc <= 4 ? decode_f32_kernel<D, V4, 4> : (hc <= 8 ? decode_f32_kernel<D, V4, 8> : decode_f32_kernel<D, V4, 16>);
+  if (hc <= 1) return decode_f32_kernel<D, V4, 1, W>;
+  if (hc <= 2) return decode_f32_kernel<D, V4, 2, W>;
+  return hc <= 4 ? decode_f32_kernel<D, V4, 4, W>
+                 : (hc <= 8 ? decode_f32_kernel<D, V4, 8, W> : decode_f32_kernel<D, V4, 16, W>);
 }
+template <bool W>
 KernelFn pick_f32(int D, bool vec, int hc) {
-  if (vec) return D == 64 ? pick_f32_hc<64, true>(hc) : pick_f32_hc<128, true>(hc);
-  return D == 64 ? pick_f32_hc<64, false>(hc) : pick_f32_hc<128, false>(hc);
+  if (vec) return D == 64 ? pick_f32_hc<64, true, W>(hc) : pick_f32_hc<128, true, W>(hc);
+  return D == 64 ? pick_f32_hc<64, false, W>(hc) : pick_f32_hc<128, false, W>(hc);
 }
 
-template <int D, int DT, bool STEP>
-KernelFn pick_mfma(bool vec, bool pipe, bool paged) {
+template <int D, int DT, bool STEP, bool W>
+KernelFn pick_mfma_step(bool vec, bool pipe, bool paged) {
   if (paged)
-    return pipe ? decode_mfma_kernel<D, DT, true, true, STEP, true> : decode_mfma_kernel<D, DT, true, false, STEP, true>;
+    return pipe ? decode_mfma_kernel<D, DT, true, true, STEP, true, W> : decode_mfma_kernel<D, DT, true, false, STEP, true, W>;
   if (vec || DT == HL_FP8)  // fp8 caches are tiled or paged: always vector loads
-    return pipe ? decode_mfma_kernel<D, DT, true, true, STEP> : decode_mfma_kernel<D, DT, true, false, STEP>;
-  if constexpr (DT != HL_FP8) return decode_mfma_kernel<D, DT, false, false, STEP>;
+    return pipe ? decode_mfma_kernel<D, DT, true, true, STEP, false, W> : decode_mfma_kernel<D, DT, true, false, STEP, false, W>;
+  if constexpr (DT != HL_FP8) return decode_mfma_kernel<D, DT, false, false, STEP, false, W>;
   return nullptr;
 }
 
-template <int D, int DT>
-KernelFn pick_mfma(bool vec, bool pipe, bool step, bool paged) {
-  return step ? pick_mfma<D, DT, true>(vec, pipe, paged) : pick_mfma<D, DT, false>(vec, pipe, paged);
+template <int DT, bool W>
+KernelFn pick_mfma(int D, bool vec, bool pipe, bool step, bool paged) {
+  if (D == 64) return step ? pick_mfma_step<64, DT, true, W>(vec, pipe, paged) : pick_mfma_step<64, DT, false, W>(vec, pipe, paged);
+  return step ? pick_mfma_step<128, DT, true, W>(vec, pipe, paged) : pick_mfma_step<128, DT, false, W>(vec, pipe, paged);
 }
 
-KernelFn pick_kernel(int kv_dtype, int D, bool vec, bool pipe, bool step, int hc, bool paged) {
-  if (kv_dtype == HL_F32) return pick_f32(D, vec, hc);
-  if (kv_dtype == HL_F16)
-    return D == 64 ? pick_mfma<64, HL_F16>(vec, pipe, step, paged) : pick_mfma<128, HL_F16>(vec, pipe, step, paged);
-  if (kv_dtype == HL_FP8)
-    return D == 64 ? pick_mfma<64, HL_FP8>(vec, pipe, step, paged) : pick_mfma<128, HL_FP8>(vec, pipe, step, paged);
-  return D == 64 ? pick_mfma<64, HL_BF16>(vec, pipe, step, paged) : pick_mfma<128, HL_BF16>(vec, pipe, step, paged);
+template <bool W>
+KernelFn pick_kernel_w(int kv_dtype, int D, bool vec, bool pipe, bool step, int hc, bool paged) {
+  if (kv_dtype == HL_F32) return pick_f32<W>(D, vec, hc);
+  if (kv_dtype == HL_F16) return pick_mfma<HL_F16, W>(D, vec, pipe, step, paged);
+  if (kv_dtype == HL_FP8) return pick_mfma<HL_FP8, W>(D, vec, pipe, step, paged);
+  return pick_mfma<HL_BF16, W>(D, vec, pipe, step, paged);
+}
+
+// wide: the kernel that folds more than 8 splits (a kernel of its own, since
+// the code alone cost the others 0.1 us of 7).
+KernelFn pick_kernel(int kv_dtype, int D, bool vec, bool pipe, bool step, int hc, bool paged, bool wide) {
+  return wide ? pick_kernel_w<true>(kv_dtype, D, vec, pipe, step, hc, paged)
+              : pick_kernel_w<false>(kv_dtype, D, vec, pipe, step, hc, paged);
 }
 
 // Resident workgroups of a kernel on the whole device (cached).
@@ -1119,7 +1174,7 @@ void decode_plan(const hl_decode_args* a, DecodePlan* plan, bool step) {
     // 2K columns: 64 one-tile splits, 27.8 us, against 16 splits, 15.2 us).
     plan->pipe = false;
     const long long fill = capacity(pick_kernel(a->kv_dtype, a->head_dim, plan->vec, false, plan->step,
-                                                plan->head_chunk, a->kv_layout == HL_KV_PAGED32)) / units;
+                                                plan->head_chunk, a->kv_layout == HL_KV_PAGED32, false)) / units;
     S = clamp_splits(mfma ? std::min<long long>(fill, std::max(1, tiles / 4)) : fill);
   }
   if (S > kMaxFusedSplits) S = kMaxFusedSplits;
@@ -1193,7 +1248,7 @@ hipError_t decode_launch(const hl_decode_args* a, const DecodePlan* plan, void* 
 
   dim3 grid(plan->num_splits, a->n_head_kv * plan->n_chunks, a->batch);
   KernelFn fn = pick_kernel(a->kv_dtype, D, plan->vec, plan->pipe, plan->step, plan->head_chunk,
-                            a->kv_layout == HL_KV_PAGED32);
+                            a->kv_layout == HL_KV_PAGED32, plan->num_splits > 8);
   hipLaunchKernelGGL(fn, grid, dim3(256), 0, stream, p);
   return hipGetLastError();
 }

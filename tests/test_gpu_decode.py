@@ -302,3 +302,31 @@ def test_decode_dropin_shape_changes_share_library_workspace(hl, orc):
         torch.cuda.synchronize()
         ref = oracle_decode(orc, q, kb, vb, 1, hq, hkv, d, [L], max_len, 0)
         assert rel_err(dst.cpu().numpy(), ref) < TOL_F32, (hq, hkv)
+
+
+# The fold of more than 8 splits: 16 a trip, and with 128 output elements or
+# fewer a workgroup, groups of threads that share the splits (1, 3 and 8 heads
+# a workgroup; remainders of 16 and of the groups; the default split counts of
+# long single sequences).  Bound: fp32 1e-5; 16-bit caches are read exactly, so
+# theirs is the same but for the 16-bit hi/lo parts of q and p (2^-16 each).
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hq,hkv,D,L,splits", [(2, 2, 64, 1100, 9), (2, 2, 64, 1100, 17), (6, 2, 64, 2100, 16),
+                                               (6, 2, 64, 2100, 33), (2, 2, 128, 3300, 50), (16, 2, 128, 2100, 31),
+                                               (8, 1, 64, 8200, 128), (2, 1, 64, 8300, 256), (32, 8, 128, 4000, 0)])
+def test_fold_of_many_splits(hl, dtype, hq, hkv, D, L, splits):
+    from hippo_leap_amd import attention as A
+    print(f"decode fold {dtype} hq={hq} hkv={hkv} D={D} L={L} splits={splits}", flush=True)
+    M = (L + 31) // 32 * 32
+    g = torch.Generator(device="cuda").manual_seed(L + splits)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    q, k, v = rnd(hq, D), rnd(hkv * D, M).to(dtype), rnd(hkv * D, M).to(dtype)
+    k[:, L:], v[:, L:] = float("nan"), float("nan")  # past the sequence: must not be used
+    out = torch.empty(hq * D, device="cuda")
+    a = A.decode_args(q, k, v, out, hq, hkv, D, M, L, num_splits=splits)
+    A.attn_decode(a, A.decode_workspace(a))
+    torch.cuda.synchronize()
+    kd, vd = (t.double().view(hkv, D, M)[:, :, :L].repeat_interleave(hq // hkv, 0) for t in (k, v))
+    p = (torch.bmm(q.double()[:, None], kd.contiguous()) / D ** 0.5).softmax(-1)
+    ref = (vd * p).sum(-1).reshape(-1)
+    err = ((out.double() - ref).abs().max() / ref.abs().max()).item()
+    assert err < (1e-5 if dtype == torch.float32 else 1e-4), err
