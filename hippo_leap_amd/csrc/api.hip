@@ -1036,11 +1036,6 @@ int hl_gpu_attention_prefill(float* dst, const float* q, const float* k, const f
   return hl_attn_prefill(&a, w.ptr, w.bytes, stream);
 }
 
-static bool overlaps(const void* a, size_t abytes, const void* b, size_t bbytes) {
-  const uintptr_t a0 = (uintptr_t)a, b0 = (uintptr_t)b;
-  return a0 < b0 + bbytes && b0 < a0 + abytes;
-}
-
 int hl_gpu_linear_col(float* dst, const float* x, const float* w, int w_cols, int w_rows,
                       int seq_len, void* stream) {
   if (!dst || !x || !w) return fail(HL_EINVAL, "linear_col: null pointer");

@@ -255,6 +255,12 @@ bool linear_quant_norm_launch(int nmat, const void* const* w, float* const* y, c
                               float* xsum, const float* x, const float* res, const float* nrm, float eps,
                               hipStream_t stream);
 
+// Whether two buffers share a byte.
+inline bool overlaps(const void* a, size_t abytes, const void* b, size_t bbytes) {
+  const uintptr_t a0 = (uintptr_t)a, b0 = (uintptr_t)b;
+  return a0 < b0 + bbytes && b0 < a0 + abytes;
+}
+
 // Sets the thread's hl_last_error() message (printf format); returns code.
 int set_error(int code, const char* fmt, ...);
 

@@ -228,10 +228,18 @@ struct DecodeFlow {
   float* S;
   float* T;
   const float* res;
+  bool apart;  // no two of the buffers overlap; otherwise nothing is folded and the plain entry points refuse
   float *q, *k, *v, *att, *o;  // this layer's projections, attention output and O projection
 
   DecodeFlow(const hl_model_desc* m_, float* x_, float* xn_, float* t0_, float* t1_, float* t2_, void* st)
-      : m(m_), x(x_), xn(xn_), t0(t0_), t1(t1_), t2(t2_), stream(st), S(x_), T(xn_), res(nullptr) {}
+      : m(m_), x(x_), xn(xn_), t0(t0_), t1(t1_), t2(t2_), stream(st), S(x_), T(xn_), res(nullptr) {
+    const size_t E = m->n_emb, q = (size_t)m->n_head * m->head_dim, kv = (size_t)m->n_head_kv * m->head_dim;
+    const size_t ff = m->n_ff, n[5] = {E, std::max(E, q), std::max({E, q, ff}), std::max(kv, ff), std::max(kv, ff)};
+    const float* const b[5] = {x, xn, t0, t1, t2};
+    apart = true;
+    for (int i = 0; i < 5; ++i)
+      for (int j = 0; j < i; ++j) apart = apart && !overlaps(b[i], n[i] * 4, b[j], n[j] * 4);
+  }
 
   // x = S + res, xn = rmsnorm(x) * weight, by a launch of its own.
   int norm(const float* weight) {
@@ -255,7 +263,7 @@ struct DecodeFlow {
     const hl_layer_desc& L = m->layers[l];
     const int E = m->n_emb, qdim = m->n_head * m->head_dim, kvdim = m->n_head_kv * m->head_dim;
     const int at = (std::max(E, qdim) + 63) / 64 * 64;
-    if (res && L.wq_type != 0 && L.wq_type == L.wk_type && L.wq_type == L.wv_type &&
+    if (apart && res && L.wq_type != 0 && L.wq_type == L.wk_type && L.wq_type == L.wv_type &&
         std::max({E, qdim, m->n_ff}) >= at + qdim && std::max(kvdim, m->n_ff) >= E) {
       const void* const ws[3] = {L.wq, L.wk, L.wv};
       float* const ys[3] = {t0 + at, t1, t2};
@@ -282,7 +290,7 @@ struct DecodeFlow {
     const int E = m->n_emb, qdim = m->n_head * m->head_dim;
     HL_TRY(linear_t(o, att, L.wo, L.wo_type, qdim, E, 1, stream));
     res = o;
-    if (L.w_gate_type == L.w_up_type &&
+    if (apart && L.w_gate_type == L.w_up_type &&
         folded(linear_quant_gate_up_norm_launch(t2, T, S, res, L.ffn_norm, m->rms_eps, L.w_gate, L.w_up, E, m->n_ff,
                                                 L.w_gate_type, (hipStream_t)stream))) {
       if (hipGetLastError() != hipSuccess) return set_error(HL_EHIP, "fused norm gate/up launch failed");
@@ -303,10 +311,11 @@ struct DecodeFlow {
   int head(float* logits, int32_t* next) {
     const void* const ws[1] = {m->output};
     float* const ys[1] = {logits};
-    const uintptr_t lo = (uintptr_t)logits, hi = lo + (size_t)m->n_vocab * 4;
-    const auto apart = [&](const float* p) { return (uintptr_t)(p + m->n_emb) <= lo || hi <= (uintptr_t)p; };
+    const size_t nb = (size_t)m->n_emb * 4, lb = (size_t)m->n_vocab * 4;
+    const auto clear = [&](const void* p, size_t bytes) { return !overlaps(logits, lb, p, bytes); };
     // logits may lie in the scratch that the unfolded launches are done with
-    if (m->output_type != 0 && apart(S) && apart(T) && apart(res) &&
+    if (apart && m->output_type != 0 && clear(S, nb) && clear(T, nb) && clear(res, nb) &&
+        clear(m->output, (size_t)quant_row_bytes(m->output_type, m->n_emb) * m->n_vocab) &&
         folded(linear_quant_norm_launch(1, ws, ys, &m->n_vocab, m->output_type, m->n_emb, T, S, res, m->output_norm,
                                         m->rms_eps, (hipStream_t)stream))) {
       if (hipGetLastError() != hipSuccess) return set_error(HL_EHIP, "fused norm output projection launch failed");
@@ -545,6 +554,14 @@ static int check_workspace(const hl_forward_scratch* s, size_t need) {
 // One launch of the fp32 projections that share x (LinearCall); a single
 // column goes through the GEMVs, a residual (onto y[0] itself) by way of tmp.
 static int prefill_linear(const LinearCall& c, void* stream, float* tmp = nullptr) {
+  // The refusals of hl_gpu_linear_col, tmp included.
+  const size_t xb = (size_t)c.K * c.T * 4;
+  for (int i = 0; i < c.nmat; ++i) {
+    const size_t yb = (size_t)c.rows[i] * c.T * 4;
+    for (const float* y : {c.pair ? c.y[0] : c.y[i], tmp})
+      if (y && (overlaps(y, yb, c.x, xb) || overlaps(y, yb, c.w[i], (size_t)c.rows[i] * c.K * 4)))
+        return set_error(HL_EINVAL, "linear_col: dst overlaps x or w");
+  }
   if (c.T > 1) {
     const hipError_t e = linear_cols_launch(c, (hipStream_t)stream);
     return e == hipSuccess ? HL_OK : set_error(HL_EHIP, "prefill linear launch: %s", hipGetErrorString(e));

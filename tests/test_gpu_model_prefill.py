@@ -270,3 +270,43 @@ def test_prefill_merged_launches(hl, E, H, Hkv, ff, T, wide):
         x = x + w["w_down"] @ (torch.nn.functional.silu(w["w_gate"] @ xn) * (w["w_up"] @ xn))
     ref = out.double() @ norm(x, onorm)
     assert rel_err(logits.cpu(), ref.cpu()) < TOL_F32
+
+
+# Scratch buffers that overlap are refused as the projections' own entry
+# points refuse them, also where one launch covers several of those calls.
+@pytest.mark.parametrize("T", [1, 5])
+@pytest.mark.parametrize("buf,onto", [("tmp0", "x_norm"), ("tmp1", "x_norm"), ("tmp2", "x_norm"), ("tmp2", "tmp0")])
+def test_prefill_refuses_overlapping_scratch(hl, orc, T, buf, onto):
+    from hippo_leap_amd import _lib
+    from hippo_leap_amd.model import DenseModel
+    print(f"prefill overlapping scratch {buf} -> {onto} T={T}", flush=True)
+    dev, _ = _build(orc, CFG, {}, False, 7)
+    m = DenseModel(torch, CFG, dev["tok_emb"], dev["output_norm"], dev["output"], 0, dev["layers"], max_tokens=8)
+    setattr(m.fscratch, buf, getattr(m.fscratch, onto))
+    with pytest.raises(_lib.HLError, match="overlap|alias"):
+        m.prefill(list(range(T)))
+    torch.cuda.synchronize()
+
+
+def test_decode_refuses_overlapping_norm_buffer(hl):
+    """x_norm on x: the residual norm refuses it, also at a size whose Q/K/V
+    and gate/up launches could take the norm in."""
+    from hippo_leap_amd import _lib
+    from hippo_leap_amd.model import DenseModel
+    E, ff, V = 2048, 2048, 64
+    cfg = dict(n_layer=2, n_emb=E, n_head=32, n_head_kv=8, head_dim=64, rope_dim=64, n_ff=ff, n_vocab=V, max_len=32,
+               rms_eps=1e-6, rope_base=1e4)
+    rows = {"wq": 2048, "wk": 512, "wv": 512, "wo": E, "w_gate": ff, "w_up": ff, "w_down": E}
+    layers = []
+    for _ in range(2):
+        L = {n: torch.zeros(r, E // 256 * 144, dtype=torch.uint8, device="cuda") for n, r in rows.items()}
+        L.update({n + "_type": _lib.HL_GGML_Q4_K for n in rows})
+        L["attn_norm"], L["ffn_norm"] = (torch.ones(E, device="cuda") for _ in range(2))
+        L["k_cache"], L["v_cache"] = (torch.zeros(512, 32, device="cuda") for _ in range(2))
+        layers.append(L)
+    m = DenseModel(torch, cfg, torch.randn(V, E, device="cuda"), torch.ones(E, device="cuda"),
+                   torch.zeros(V, E, device="cuda"), 0, layers)
+    m.fscratch.x_norm = m.fscratch.x
+    with pytest.raises(_lib.HLError, match="norm_out overlaps x"):
+        m.decode()
+    torch.cuda.synchronize()
