@@ -56,19 +56,26 @@ __global__ __launch_bounds__(256) void rmsnorm_col_kernel(const float* __restric
 // used).  out may be x.
 //
 // Bound by the latency of one pass over few columns: the walk down a column
-// must be short, since seq / CB workgroups are all there are.  64 columns per
-// 256-thread workgroup (512 dependent-load rounds per thread at dim 2048, 5
-// workgroups at 301 columns) took 172 us for 2048 x 301; 8 columns: 9.1 us.
-// 16 columns (64-byte segments) from 2048 columns on, where the grid has a
-// workgroup for half of the CUs anyway (4096 x 4096: 51 us against 82 with 8;
-// 647 with 64).
+// must be short, since seq / CB workgroups are all there are.  The workgroups
+// of adjacent columns share a row's cache lines, so each XCD takes a run of
+// them.  us with 64 columns per 256-thread workgroup, then with 8 (16 from
+// 2048 on) in launch order, now:
+//   2048 x 301   172   9.0   6.9      4096 x 1000  556  20.1  13.9
+//   4096 x 512         16.6  11.8     4096 x 4096  647  51.8  37.5
+//   4096 x 37 (one column per workgroup) 12.6, now 11.0; 4096 x 7 6.6, now 5.2
+// Columns per workgroup, same order of workgroups, 2 / 4 / 8 / 16:
+//   2048 x 301  6.8  6.9  8.1 | 4096 x 512  13.2 11.8 14.0 | 4096 x 1000 21.8 13.9 15.0
+//   4096 x 2000  26.3 (4) 19.6 (8) | 4096 x 2900  41.8 (8) 36.4 (16) | 4096 x 4096  43.7 (8) 37.5 (16)
+// hence 4 up to 1024 columns, 8 below 2048, 16 from there on.
 template <int CB, int NR>
 __global__ __launch_bounds__(1024) void norm_cols_kernel(const float* x, const float* __restrict__ w, float* out,
                                                          int dim, int seq, float eps) {
   constexpr int G = 1024 / CB;
   __shared__ float part[16][CB];
   const int c = threadIdx.x % CB, g = threadIdx.x / CB;
-  const int col = blockIdx.x * CB + c;
+  // Workgroup id mod 8 is the XCD.
+  const int xcd = blockIdx.x % 8, rem = gridDim.x % 8;
+  const int col = (xcd * (int)(gridDim.x / 8) + min(xcd, rem) + (int)blockIdx.x / 8) * CB + c;
   const size_t cc = min(col, seq - 1);
   float v[NR], ss = 0.f;
 #pragma unroll
@@ -183,8 +190,12 @@ hipError_t rmsnorm_cols_launch(float* out, const float* x, const float* w, int d
   if (seq == 1 && vec4_ok(dim, x, w, out, out))
     hipLaunchKernelGGL(norm_vec4_kernel<false>, dim3(1), dim3(1024), 0, stream, const_cast<float*>(x), x,
                        nullptr, w, out, dim, eps);
-  else if (seq < 64)  // 4096 x 37: 9.4 us against 9.5, x 7: 6.8 against 7.8
+  else if (seq == 1 || (seq < 16 && dim < 1024))  // 512 x 5: 2.4 us against 2.7 with 4 columns; 2048 x 3: 3.8, 3.4
     hipLaunchKernelGGL(rmsnorm_col_kernel, dim3(seq), dim3(256), 0, stream, x, w, out, dim, seq, eps);
+  else if (seq <= 1024 && dim <= 2048)
+    hipLaunchKernelGGL((norm_cols_kernel<4, 8>), dim3((seq + 3) / 4), dim3(1024), 0, stream, x, w, out, dim, seq, eps);
+  else if (seq <= 1024)
+    hipLaunchKernelGGL((norm_cols_kernel<4, 16>), dim3((seq + 3) / 4), dim3(1024), 0, stream, x, w, out, dim, seq, eps);
   else if (seq >= 2048)
     hipLaunchKernelGGL((norm_cols_kernel<16, 32>), dim3((seq + 15) / 16), dim3(1024), 0, stream, x, w, out, dim, seq, eps);
   else if (dim <= 2048)

@@ -61,10 +61,12 @@ def test_residual_rmsnorm_misaligned(hl, orc):
     assert rel_err(out.cpu().numpy(), orc.rmsnorm(xs.reshape(1, dim), w, 1e-6).reshape(-1)) < TOL_F32
 
 
-@pytest.mark.parametrize("dim,T", [(2048, 301), (2049, 65), (4097, 71), (127, 66), (9001, 129), (96, 2048), (2050, 2063)])
+@pytest.mark.parametrize("dim,T", [(2048, 301), (2049, 65), (4097, 71), (127, 66), (9001, 129), (96, 2048), (2050, 2063),
+                                   (1024, 2), (1023, 16), (2048, 5), (4097, 37), (2049, 1024), (2048, 1025),
+                                   (2049, 1031), (9001, 2047)])
 def test_rmsnorm_cols_of_a_prompt(hl, dim, T):
-    """The kernel that keeps a thread's rows in registers (T >= 64): around
-    its row groups, more rows than it keeps, both column counts, in place.
+    """The kernel that keeps a thread's rows in registers (T >= 2): around
+    its row groups, more rows than it keeps, each column count, in place.
     Bound: the sum of squares and three roundings, (dim / 64 + 16) 2^-24."""
     from hippo_leap_amd import attention as A
     print(f"rmsnorm_cols prompt dim={dim} T={T}", flush=True)
