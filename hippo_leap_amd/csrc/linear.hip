@@ -14,9 +14,10 @@
 //   small, so the grid still covers the chip), one cross-lane reduction per
 //   row.  x is re-read from L2 by every wave (staging it in LDS measured
 //   slower).
-// * T > 1 (prefill): linear_split_kernel, three fp16 MFMAs
-//   (v_mfma_f32_32x32x16_f16) on hi/lo parts of the fp32 operands per fp32
-//   product; fp32 MFMAs for the output tiles where that is not possible.
+// * T > 1 (prefill): linear_split_kernel, six bf16 MFMAs
+//   (v_mfma_f32_32x32x16_bf16) on the three bf16 parts of the fp32 operands
+//   per fp32 product; fp32 MFMAs for the output tiles where that is not
+//   possible.
 //
 // Accumulation is fp32 as in the reference; only the summation order
 // differs (the reference's decode kernel reduces 256 strided partial sums,
@@ -106,25 +107,46 @@ __global__ __launch_bounds__(256) void linear_gemv_kernel(const float* __restric
 }
 
 // ---------------------------------------------------------------------------
-// GEMM (T > 1) on fp16 MFMA over split fp32 operands
+// GEMM (T > 1) on bf16 MFMA over split fp32 operands
 // ---------------------------------------------------------------------------
-// Every operand x becomes x s = hi + lo, hi = f16(x s), lo = f16(x s - hi),
-// s a power of two per row of W and per column of X; a product is then
-// hi hi' + hi lo' + lo hi' into one fp32 accumulator (lo lo' is below 2^-22
-// of it).  That costs 3 x 32 matrix-core cycles per 32x32x16 block where
-// v_mfma_f32_32x32x2_f32 takes 8 x 64.  Error: 2^-23 of each element and
-// 2^-25 absolute after scaling (the MFMA takes f16 subnormals as they are),
-// below the fp32 accumulation's own: against a 64-bit product
-// 2.6e-7 at K = 4096 and 2.0e-7 at 2048 where fp32 MFMAs gave 1.1e-6 and
-// 4.1e-7 (one accumulation chain of K instead of KW chains of 16-long sums).
+// Every operand x is the sum of three bf16 numbers, each the rounded rest of
+// the one before: p0 = bf16(x), p1 = bf16(x - p0), p2 = x - p0 - p1.  bf16 has
+// the exponents of fp32, so this needs no scale and holds all 24 bits of any
+// element, however large its neighbours are.  A product is the six products of
+// parts p0 p2', p2 p0', p1 p1', p0 p1', p1 p0', p0 p0'; the three left out are
+// at most 2^-24 of it, the rounding of one fp32 product.  The matrix cores
+// take bf16 subnormals, and give fp32 ones, as they are (test_small_parts).
 //
-// s brings the largest magnitude of the first 16 k that a wave meets into
-// [64, 128): the absolute error is then 2^-31 of it, and later elements may
-// be 2^9 times larger.  One above that, an inf or a NaN makes a partial sum
-// inf or NaN, and the workgroup then computes its tile once more with fp32
-// MFMAs (body<false>), so that inf and NaN come out as fp32 arithmetic gives
-// them.  A row or column whose first 16 elements are
-// zero is scanned for its largest element instead.
+// Bits below the smallest bf16 subnormal (of elements below 2^-109) are the
+// only ones that the parts miss: the rests are collected, and a workgroup that
+// has met one, or whose partial sums hold an inf or a NaN, computes its tile
+// once more with fp32 MFMAs (body<false>), so that those come out as fp32
+// arithmetic gives them.  Nothing else goes there: two f16 parts and a scale
+// from a row's first elements (three products, 1.3 to 1.5 times as fast) lost
+// elements 2^14 and more below those, and did every tile twice that met one
+// 2^9 above them.
+//
+// Cost: 6 x 32 matrix-core cycles per 32x32x16 block where
+// v_mfma_f32_32x32x2_f32 takes 8 x 64, and 6 VALU instructions per element
+// and lane, spread part by part over the MFMAs of the blocks before (in bursts
+// of a whole split: 14336 x 4096, 1000 columns 681 us, so 618).
+// v_dot2_f32_bf16, which would halve the subtractions, took twice the time in
+// all and did not subtract exactly.
+//
+// The small products have sums of their own: an MFMA cuts what lies below the
+// last place of its largest addend towards minus infinity, so that small
+// products (and a full fp32 sum added to larger products) shift every output
+// the same way, by 1e-7 of their spread, which the layers of a model add up
+// (Llama-3.2-1B, 16 layers, logits against 64 bits: 2.0e-6, now 7.7e-7; fp32
+// MFMAs 2.1e-6).  Large
+// products lose nothing in acc.  CROSS keeps accumulators of the small ones over
+// all of K; the 64x64 tiles have no registers for those and sum a block's five
+// small products of 16 k, which the VALU adds to acc behind the next block's
+// MFMAs.  Error against a 64-bit product: 1.3e-7 at K = 2048, 1.4e-7 to 1.9e-7 at
+// 4096, 3.7e-7 at 14336, where all six into one accumulator gave 2.5e-7, 3.5e-7
+// to 5.0e-7 and 9.9e-7, and fp32 MFMAs in one chain of K 4.1e-7 at 2048 and
+// 1.1e-6 at 4096.  The sums by VALU cost 7 to 10% (2048 x 8192, 301 columns: 82
+// -> 91 us; added at the end of their own block: 97), CROSS 2%.
 //
 // The KW waves of a workgroup share one (32 WM) x (32 WN) output tile and
 // split K between them in chunks of CK (wave w takes chunks w, w + KW, ...),
@@ -134,33 +156,31 @@ __global__ __launch_bounds__(256) void linear_gemv_kernel(const float* __restric
 // registers, XD 16-k steps ahead: lane ln of a half holds columns
 // WN ln .. WN ln + WN - 1 of 8 k, so one load of 4 WN bytes serves the WN
 // column blocks, and neither K nor T nor an address has to be a multiple of
-// anything.  The splits cost 2 (multiply) + 2 (v_cvt_pk_f16_f32) + 4
-// (v_fma_mix_f32) + 2 cycles per element and lane; v_fma_mixlo_f16, which
-// would take two instructions, measured 8 cycles each.  The splits of the next
-// column block and of the next step's rows stand between the MFMAs of this
-// one: 3 to 5% over splitting a block and then multiplying it (14336 x 4096,
-// 1000: 481 -> 464 us; 4096 x 14336: 459 -> 434; 4096 x 4096, 128: 34.2 -> 31.5).
+// anything.
 //
 // A launch takes up to three matrices on the same X, a residual to add, or
 // gate and up with SiLU * up on the sums: a prompt's layers then need four
 // GEMM launches for ten kernels, tiles of small matrices share a round, and
 // the sums of gate and up never go to memory.  Llama-3.2-1B shapes, 301
-// tokens, a whole prefill: 6.17 -> 5.46 ms (Q/K/V 51 -> 28 us a layer, gate,
-// up and SiLU 131 -> 105, the two additions 10 -> 0).
+// tokens, a whole prefill, when this was done: 6.17 -> 5.46 ms (Q/K/V 51 -> 28
+// us a layer, gate, up and SiLU 131 -> 105, the two additions 10 -> 0).
 //
 // What bounds it: bytes into the CUs on the small tiles (128 B per k of a
 // 64x64 tile from L2; the prefetch depth did not matter), the matrix cores
-// at three products on 64x128 tiles.  Before: fp32 MFMAs on 128x128 tiles
-// staged through LDS, scalar loads whenever K or T was no multiple of 4.
+// at six products on 64x128 tiles (1.1 PFLOP/s of bf16).  Before: fp32 MFMAs on
+// 128x128 tiles staged through LDS, scalar loads whenever K or T was no
+// multiple of 4.
 //   M x K, T              before      now
-//   4096 x 4096,    37    130 us     19.9   (32x32 tiles)
-//   2048 x 2048,   301     76        20.4   (64x64)
-//   2048 x 8192,   301    267        62     (64x64)
-//   14336 x 4096, 1000   1080       464     (64x128: 253 TFLOP/s)
-//   4096 x 4096,  4096   1044       522     (64x128: 263 TFLOP/s)
+//   4096 x 4096,    37    130 us     28     (32x32 tiles)
+//   2048 x 2048,   301     76        28     (64x64)
+//   2048 x 8192,   301    267        91     (64x64)
+//   14336 x 4096, 1000   1080       650     (64x128: 181 TFLOP/s)
+//   4096 x 4096,  4096   1044       728     (64x128: 189 TFLOP/s)
+// (14336 x 4096, 1000, with a NaN in every tile, so that all are computed twice:
+// 1530 us.)
 // Measured and not kept: x loads four steps ahead (no change), 64-k chunks on
-// 64x64 tiles (17% slower), sixteen waves (slower), 128x64 and 128x128 tiles.
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+// 64x64 tiles (17% slower), sixteen waves (slower), 128x64 and 128x128 tiles;
+// sums by VALU on 64x128 tiles (784 us instead of 650).
 
 // N floats at a 4-byte aligned address.
 template <int N>
@@ -178,45 +198,49 @@ __device__ __forceinline__ void load_n(const float* p, float* v) {
   }
 }
 
-// x s - hi in fp32, hi the low (J = 0) or high half of a packed f16 pair.
-template <int J>
-__device__ __forceinline__ float split_rest(float x, float s, uint32_t hi) {
-  float r;
-  if constexpr (J == 0) asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(r) : "v"(x), "v"(s), "v"(hi));
-  else asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(r) : "v"(x), "v"(s), "v"(hi));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+// Two values rounded to bf16; through an empty asm, or the compiler would
+// convert once more for each use of a half.
+__device__ __forceinline__ uint32_t pack_bf16(float v0, float v1) {
+  uint32_t r = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)v0, (__bf16)v1});
+  asm("" : "+v"(r));
   return r;
 }
-__device__ __forceinline__ uint32_t pack_f16(float a, float b) {
-  return __builtin_bit_cast(uint32_t, f16x2{(_Float16)a, (_Float16)b});
-}
-__device__ __forceinline__ void split2(float v0, float v1, float s, uint32_t& hi, uint32_t& lo) {
-  hi = pack_f16(v0 * s, v1 * s);
-  lo = pack_f16(split_rest<0>(v0, s, hi), split_rest<1>(v1, s, hi));
-}
+// Parts 0 (largest) to 2 of eight values.
 struct Split8 {
-  u32x4 hi, lo;
+  u32x4 part[3];
 };
-__device__ __forceinline__ f16x8 as_f16(const u32x4& v) { return __builtin_bit_cast(f16x8, v); }
-__device__ __forceinline__ Split8 split8(const float* v, float s) {
+__device__ __forceinline__ bf16x8 as_bf16(const u32x4& v) { return __builtin_bit_cast(bf16x8, v); }
+// Part i of a pair of values, j of the eight; leaves what is below it in v.
+// lost collects the bits that are in no part.
+struct Pair {
+  float v0, v1;
+};
+__device__ __forceinline__ void split_part(Pair& v, Split8& r, int j, int i, uint32_t& lost) {
+  const uint32_t h = pack_bf16(v.v0, v.v1);
+  r.part[i][j] = h;
+  if (i < 2) {
+    v.v0 -= __uint_as_float(h << 16);
+    v.v1 -= __uint_as_float(h & 0xFFFF0000u);
+  } else {
+    // In asm, so that the collection is not put off (the rests of a whole
+    // step would be live, which spills).
+    asm("v_or3_b32 %0, %1, %2, %0" : "+v"(lost) : "v"(v.v0), "v"(v.v1));
+  }
+}
+__device__ __forceinline__ Split8 split8(const float* v, uint32_t& lost) {
   Split8 r;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    uint32_t h, l;
-    split2(v[2 * j], v[2 * j + 1], s, h, l);
-    r.hi[j] = h;
-    r.lo[j] = l;
+    Pair p = {v[2 * j], v[2 * j + 1]};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) split_part(p, r, j, i, lost);
   }
   return r;
 }
-
-// The power of two that brings magnitude m into [64, 128) (1 for m = 0).  bad:
-// m is outside 2^-100 .. 2^100, inf or NaN.
-__device__ __forceinline__ float split_scale(float m, bool& bad) {
-  const uint32_t e = __float_as_uint(m) >> 23;
-  if (m == 0.f) return 1.f;
-  bad = bad || e < 27u || e > 227u;
-  return __uint_as_float((260u - e) << 23);
-}
+// The six products of parts that are kept, smallest first.
+constexpr int kProducts = 6;
+constexpr int kPartA[kProducts] = {0, 2, 1, 0, 1, 0}, kPartB[kProducts] = {2, 0, 1, 1, 0, 0};
 
 // Orders a wave's LDS writes and reads (each wave has its own staging area).
 __device__ __forceinline__ void wave_lds_sync() {
@@ -240,7 +264,7 @@ struct SplitArgs {
 // rows of a tile are 16 of gate and the same 16 of up, which meet in one lane
 // of the final sums.  Otherwise the row tiles run over the matrices in order.
 template <int WM, int WN, int KW, int CK, int XD, bool PAIR>
-__global__ __launch_bounds__(64 * KW) void linear_split_kernel(SplitArgs p) {
+__global__ __launch_bounds__(64 * KW, WM * WN == 8 ? 1 : 2) void linear_split_kernel(SplitArgs p) {
   constexpr int ST = CK / 16;            // 16-k steps per chunk
   constexpr int BM = 32 * WM, BN = 32 * WN;
   constexpr int C16 = CK / 4;            // 16-byte pieces per staged row
@@ -248,9 +272,12 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(SplitArgs p) {
   constexpr int RPL = 64 / C16;          // rows per load
   constexpr int STAGE = BM * CK;         // floats of a wave's staging area
   constexpr int PART = BM * BN;          // floats of a wave's partial sums
+  // The 64x64 tiles have 256 registers a wave: no accumulators for the small
+  // products, and the next step's rows are split behind this one's MFMAs (a
+  // second wave on the SIMD has MFMAs meanwhile; 2 to 3%).
+  constexpr bool CROSS = WM * WN != 4, PIPE_A = CROSS;
   static_assert(XD <= ST && ST % XD == 0, "x buffers");
   __shared__ __attribute__((aligned(16))) float lds[KW * (STAGE > PART ? STAGE : PART)];
-  __shared__ __attribute__((aligned(16))) float inv_row[KW][BM];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -296,7 +323,7 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(SplitArgs p) {
   f32x16 acc[WM][WN];
 
   // This wave's share of K into acc, on split operands or (false) on fp32
-  // MFMAs.  Returns true when the split operands cannot hold a value.
+  // MFMAs.  Returns true when the parts do not hold every bit of a value.
   auto body = [&](auto split_tag) -> bool {
     constexpr bool SPLIT = decltype(split_tag)::value;
 #pragma unroll
@@ -307,7 +334,13 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(SplitArgs p) {
         for (int e = 0; e < 16; ++e) acc[a][b][e] = 0.f;
     f32x4 wr[NL];
     float xr[XD][8][WN];
-    [[maybe_unused]] float sa[WM], sb[WN];
+    [[maybe_unused]] uint32_t lost = 0;
+    [[maybe_unused]] f32x16 cross[WM][WN], sums = {}, done;
+    if constexpr (SPLIT && CROSS)
+#pragma unroll
+      for (int a = 0; a < WM; ++a)
+#pragma unroll
+        for (int b = 0; b < WN; ++b) cross[a][b] = f32x16{};
     auto load_w = [&](int c) {
       const float* src = wt + (size_t)c * CK;
       [[maybe_unused]] const float* src2 = PAIR ? wt2 + (size_t)c * CK : nullptr;
@@ -335,74 +368,48 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(SplitArgs p) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) v[j] = v0[j], v[4 + j] = v1[j];
     };
-    auto scales = [&](const float (*xv)[WN]) -> bool {
-      float ma[WM], mb[WN];
-      bool zero = false, bad = false;
-#pragma unroll
-      for (int a = 0; a < WM; ++a) {
-        float v[8];
-        read_a(a, 0, v);
-        ma[a] = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ma[a] = fmaxf(ma[a], fabsf(v[j]));
-        ma[a] = fmaxf(ma[a], __shfl_xor(ma[a], 32, 64));
-        zero = zero || ma[a] == 0.f;
-      }
-#pragma unroll
-      for (int b = 0; b < WN; ++b) {
-        mb[b] = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) mb[b] = fmaxf(mb[b], fabsf(xv[j][b]));
-        mb[b] = fmaxf(mb[b], __shfl_xor(mb[b], 32, 64));
-        zero = zero || mb[b] == 0.f;
-      }
-      if (__any(zero)) {  // rare: the largest elements of this wave's whole share
-        for (int c = wave; c * CK < K; c += KW)
-          for (int k = c * CK + hh; k < min(c * CK + CK, K); k += 2) {
-#pragma unroll
-            for (int a = 0; a < WM; ++a)
-              ma[a] = fmaxf(ma[a], fabsf(wbase(ln)[(size_t)wrow(32 * a + ln) * K + k]));
-#pragma unroll
-            for (int b = 0; b < WN; ++b) mb[b] = fmaxf(mb[b], fabsf(x[(size_t)k * T + col0 + b]));
-          }
-#pragma unroll
-        for (int a = 0; a < WM; ++a) ma[a] = fmaxf(ma[a], __shfl_xor(ma[a], 32, 64));
-#pragma unroll
-        for (int b = 0; b < WN; ++b) mb[b] = fmaxf(mb[b], __shfl_xor(mb[b], 32, 64));
-      }
-#pragma unroll
-      for (int a = 0; a < WM; ++a) {
-        sa[a] = split_scale(ma[a], bad);
-        if (hh == 0) inv_row[wave][32 * a + ln] = 1.0f / sa[a];
-      }
-#pragma unroll
-      for (int b = 0; b < WN; ++b) sb[b] = split_scale(mb[b], bad);
-      wave_lds_sync();
-      return __any(bad);
+    auto split_a = [&](int a, int s, Split8* A) {
+      float v[8];
+      read_a(a, s, v);
+      A[a] = split8(v, lost);
     };
     auto split_b = [&](const float (*xv)[WN], int b) {
       float v[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = xv[j][b];
-      return split8(v, sb[b]);
+      return split8(v, lost);
     };
-    // MFMA i of the 3 WM of a column block: lo hi', hi lo', hi hi'.
-    auto product = [&](const Split8* A, const Split8& B, int b, int i) {
-      const int a = i % WM;
-      acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16(i < WM ? A[a].lo : A[a].hi),
-                                                         as_f16(i / WM == 1 ? B.lo : B.hi), acc[a][b], 0, 0, 0);
+    // The products of 16 k of column block b, work(i) behind MFMA i.
+    auto products = [&](const Split8* A, const Split8& B, int b, auto work) {
+#pragma unroll
+      for (int i = 0; i < kProducts * WM; ++i) {
+        const int a = CROSS ? i % WM : i / kProducts, q = CROSS ? i / WM : i % kProducts;
+        const bf16x8 pa = as_bf16(A[a].part[kPartA[q]]), pb = as_bf16(B.part[kPartB[q]]);
+        const bool small = q < kProducts - 1;
+        if (!CROSS && q == 0) done = sums;
+        f32x16& c = !small ? acc[a][b] : CROSS ? cross[a][b] : sums;
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa, pb, !CROSS && q == 0 ? f32x16{} : c, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        work(i);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!CROSS) {
+          const int at = (b * WM + a + WM * WN - 1) % (WM * WN);  // block that done belongs to
+#pragma unroll
+          for (int e = 16 * q / kProducts; e < 16 * (q + 1) / kProducts; ++e) acc[at % WM][at / WM][e] += done[e];
+          asm volatile("" : "+v"(acc[at % WM][at / WM]));  // here, or the sums of all blocks would be live
+        }
+      }
     };
     // Step s on operands split before (A, B of column block 0); splits those
     // of the next step (its x in xn, its A if next_a) and of the other column
     // blocks between the MFMAs.  load_next overwrites xv once it is split.
     auto piped = [&](int s, const float (*xv)[WN], const float (*xn)[WN], Split8* A, Split8& B, bool next_a,
                      auto load_next) {
-      constexpr int N = 3 * WM;
-      float va[WM][8];
+      constexpr int N = kProducts * WM;
+      float va[8];
       Split8 A2[WM];
-      if (next_a)
-#pragma unroll
-        for (int a = 0; a < WM; ++a) read_a(a, s + 1, va[a]);
+      Pair pa, pb;
+      if (PIPE_A && next_a) read_a(0, s + 1, va);
 #pragma unroll
       for (int b = 0; b < WN; ++b) {
         Split8 B2;
@@ -412,51 +419,40 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(SplitArgs p) {
           load_next();
         }
         __builtin_amdgcn_sched_barrier(0);
+        products(A, B, b, [&](int i) {
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-          product(A, B, b, i);
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int j = 4 * i / N; j < 4 * (i + 1) / N; ++j) {  // of the next column block
+          for (int u = 12 * i / N; u < 12 * (i + 1) / N; ++u) {  // of the next column block
+            const int j = u / 3, q = u % 3;
             const float(*src)[WN] = nb ? xv : xn;
-            uint32_t h, l;
-            split2(src[2 * j][nb], src[2 * j + 1][nb], sb[nb], h, l);
-            B2.hi[j] = h;
-            B2.lo[j] = l;
+            if (q == 0) pb = Pair{src[2 * j][nb], src[2 * j + 1][nb]};
+            split_part(pb, B2, j, q, lost);
           }
           const int at = b * N + i;
-          if (next_a)
+          if (PIPE_A && next_a)
 #pragma unroll
-            for (int u = 4 * WM * at / (N * WN); u < 4 * WM * (at + 1) / (N * WN); ++u) {  // of the next step's A
-              const int a = u / 4, j = u % 4;
-              uint32_t h, l;
-              split2(va[a][2 * j], va[a][2 * j + 1], sa[a], h, l);
-              A2[a].hi[j] = h;
-              A2[a].lo[j] = l;
+            for (int u = 12 * WM * at / (N * WN); u < 12 * WM * (at + 1) / (N * WN); ++u) {  // of the next step's A
+              const int a = u / 12, j = u / 3 % 4, q = u % 3;
+              if (q == 0) pa = Pair{va[2 * j], va[2 * j + 1]};
+              split_part(pa, A2[a], j, q, lost);
+              if (j == 3 && q == 2 && a + 1 < WM) read_a(a + 1, s + 1, va);
             }
-          __builtin_amdgcn_sched_barrier(0);
-        }
+        });
         B = B2;
       }
       if (next_a)
 #pragma unroll
-        for (int a = 0; a < WM; ++a) A[a] = A2[a];
+        for (int a = 0; a < WM; ++a) {
+          if constexpr (PIPE_A) A[a] = A2[a];
+          else split_a(a, s + 1, A);
+        }
     };
     auto step = [&](int s, const float (*xv)[WN]) {
       if constexpr (SPLIT) {
         Split8 A[WM];
 #pragma unroll
-        for (int a = 0; a < WM; ++a) {
-          float v[8];
-          read_a(a, s, v);
-          A[a] = split8(v, sa[a]);
-        }
+        for (int a = 0; a < WM; ++a) split_a(a, s, A);
 #pragma unroll
-        for (int b = 0; b < WN; ++b) {
-          const Split8 B = split_b(xv, b);
-#pragma unroll
-          for (int i = 0; i < 3 * WM; ++i) product(A, B, b, i);
-        }
+        for (int b = 0; b < WN; ++b) products(A, split_b(xv, b), b, [](int) {});
       } else {
         // MFMA j pairs k 8 hh + j of the two lane halves
 #pragma unroll
@@ -471,7 +467,6 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(SplitArgs p) {
         }
       }
     };
-    bool scaled = false;
     if (nmine > 0) {
       // The loads are unconditional (the last ones repeat the last chunk and
       // are not used) and kept in program order, so that every wait counts
@@ -486,18 +481,11 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(SplitArgs p) {
         __builtin_amdgcn_sched_barrier(0);
         load_w(cn);
         __builtin_amdgcn_sched_barrier(0);
-        if (SPLIT && n == 0) {
-          if (scales(xr[0])) return true;
-          scaled = true;
-          if constexpr (SPLIT) B = split_b(xr[0], 0);
-        }
-        if constexpr (SPLIT)
+        if constexpr (SPLIT) {
+          if (n == 0) B = split_b(xr[0], 0);
 #pragma unroll
-          for (int a = 0; a < WM; ++a) {
-            float v[8];
-            read_a(a, 0, v);
-            A[a] = split8(v, sa[a]);
-          }
+          for (int a = 0; a < WM; ++a) split_a(a, 0, A);
+        }
 #pragma unroll
         for (int s = 0; s < ST; ++s) {
           auto load_next = [&]() {
@@ -536,35 +524,21 @@ __global__ __launch_bounds__(64 * KW) void linear_split_kernel(SplitArgs p) {
 #pragma unroll
           for (int b = 0; b < WN; ++b) xr[0][j][b] = kb + j < K ? xr[0][j][b] : 0.f;
         }
-        if (SPLIT && !scaled) {
-          if (scales(xr[0])) return true;
-          scaled = true;
-        }
         step(s, xr[0]);
       }
     }
-    if constexpr (SPLIT) {
-      if (scaled) {  // back to the operands' own scale
+    if constexpr (SPLIT && !CROSS) acc[WM - 1][WN - 1] += sums;
+    if constexpr (SPLIT && CROSS)
 #pragma unroll
-        for (int a = 0; a < WM; ++a)
+      for (int a = 0; a < WM; ++a)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const f32x4 ir = *(const f32x4*)&inv_row[wave][32 * a + 8 * q + 4 * hh];
-#pragma unroll
-            for (int b = 0; b < WN; ++b) {
-              const float ib = 1.0f / sb[b];
-#pragma unroll
-              for (int e = 0; e < 4; ++e) acc[a][b][4 * q + e] = acc[a][b][4 * q + e] * ir[e] * ib;
-            }
-          }
-      }
-    }
-    return false;
+        for (int b = 0; b < WN; ++b) acc[a][b] += cross[a][b];
+    return (lost & 0xFFFFu) != 0;
   };
 
   // The waves' partial sums meet in LDS ([wave][a][b][q][lane], four rows
   // each) and are added in wave order.  CHECK: if one is inf or NaN (or a
-  // wave could not split) nothing is stored and the result is false.
+  // wave met bits outside its parts) nothing is stored and the result is false.
   auto finish = [&](auto check_tag, bool bad) -> bool {
     constexpr bool CHECK = decltype(check_tag)::value;
     // Units of four rows per lane: (a, q) of the tile, for PAIR q = 0, 1 (gate)
@@ -646,9 +620,9 @@ inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // The split GEMM's variants: tile, workgroups resident on a CU, and the model
 // of their time by which one is chosen, in us:
 //   2 + rounds of workgroups * (fixed + K / 1000 * (only round ? one : more)).
-// Fitted to 78 timed shapes (256 .. 14336 rows and k, 2 .. 4096 columns): the
-// choice is 0.2% off the best of the four on average, 7% at worst; always
-// taking 64x64 would cost 1.9x at 37 columns, always 32x32 2.2x at 1000.
+// On 80 timed shapes (256 .. 14336 rows and k, 2 .. 4096 columns) the choice is
+// 0.7% off the best of the four on average, 20% at worst; always taking one
+// would cost 1.35 to 1.85 times as much on average.
 struct SplitVariant {
   int bm, bn, per_cu;
   float fixed, one, more;
@@ -714,7 +688,7 @@ hipError_t linear_cols_launch(const LinearCall& c, hipStream_t stream) {
   if (p.variant == 0) launch_split<1, 1, 8, 64, 4>(a, c.pair, stream);
   else if (p.variant == 1) launch_split<2, 2, 8, 32, 2>(a, c.pair, stream);
   else if (p.variant == 2) launch_split<2, 2, 4, 32, 2>(a, c.pair, stream);
-  else launch_split<2, 4, 4, 64, 2>(a, c.pair, stream);
+  else launch_split<2, 4, 4, 32, 2>(a, c.pair, stream);
   return hipGetLastError();
 }
 

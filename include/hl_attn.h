@@ -218,7 +218,11 @@ int hl_gpu_attention_prefill(float* dst, const float* q, const float* k,
 /* gpuLinearCol (naive.nim:3519-3547), the Q/K/V and O projections around
  * attention: dst[wRows, seqLen] = w[wRows, wCols] . x[wCols, seqLen], all
  * fp32; w row-major (wCols fastest), x and dst with seqLen fastest.
- * seq_len == 1 is the decode GEMV, seq_len > 1 the prefill GEMM.  dst must
+ * seq_len == 1 is the decode GEMV, seq_len > 1 the prefill GEMM, whose
+ * products are those of each element's three bf16 parts, which hold all of
+ * its 24 bits whatever its neighbours are: per output, |error| <=
+ * (K / 10 + 48) 2^-24 sum_k |w| |x| (K = wCols; the K terms of fp32 MFMAs
+ * where an inf, a NaN or an element below 2^-109 is met).  dst must
  * not overlap x or w (HL_EINVAL: the outputs would race with the reads).
  * Unlike the reference's decode kernel there is no width cap
  * (HippoMaxDecodeCols = 18432, naive.nim:20, 3530-3533).                 */

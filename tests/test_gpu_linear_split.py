@@ -1,14 +1,16 @@
 """GPU: the split-operand GEMM of hl_gpu_linear_col (seq_len > 1) at the edges
-of its tiles, chunks and column vectors, and with operands that leave the
-range of its split (zero runs, values far above a row's first ones,
-subnormal rows, inf and NaN), against float64 products of the same inputs.
+of its tiles, chunks and column vectors, and with operands of every fp32 range
+(zero runs, elements far above and far below the others of their row, subnormal
+parts, inf and NaN), against float64 products of the same inputs.
 
-Bound: each operand is held to 2^-23 of itself and 2^-31 of the largest of a
-16-element run of its row (column), three of the four partial products are
-kept (the fourth is below 2^-22), and every 16-long sum is added to an fp32
-accumulator.  So |error| <= (2^-20 + (K / 16 + 32) 2^-24) |W| |X| + 2^-30
-(max|w| sum|x| + max|x| sum|w|) per output; a tile that falls back to fp32
-MFMAs accumulates K terms, K 2^-24 more."""
+Bound, per output and without a term in a row's or column's largest element:
+the three bf16 parts hold an element whole, the products of parts that are left
+out are at most 2^-24 of the element's product, and the six kept ones of 16 k
+are each added to an fp32 accumulator with one rounding, K split over at least
+four waves, whose sums meet in eight more.  So |error| <= (6 / 4 K / 16 + 8 +
+16 + 1) 2^-24 |W| |X|, here (K / 10 + 48) 2^-24; results below the normal range
+add 2^-149 per rounding.  A tile that goes to fp32 MFMAs accumulates K terms,
+K 2^-24 more."""
 import numpy as np
 import pytest
 import torch
@@ -32,10 +34,8 @@ def _check(w, x, fp32=False):
     y = _run(w, x)
     ref = w.double() @ x.double()
     mag = w.double().abs() @ x.double().abs()
-    bound = (2.0 ** -20 + ((K if fp32 else 0) + K / 16 + 32) * 2.0 ** -24) * mag
-    wa, xa = w.double().abs(), x.double().abs()
-    bound += 2.0 ** -30 * (wa.amax(1, True) * xa.sum(0, True) + xa.amax(0, True) * wa.sum(1, True))
-    worst = ((y.double() - ref).abs() / bound.clamp_min(1e-300)).max().item()
+    bound = ((K if fp32 else 0) + K / 10 + 48) * 2.0 ** -24 * mag + (K + 48) * 2.0 ** -149
+    worst = ((y.double() - ref).abs() / bound).max().item()
     assert worst <= 1.0, worst
 
 
@@ -60,10 +60,14 @@ def test_edges(hl, M, K, T):
         _check(*_operands(M, K, T, 17 * M + K + T, offset))
 
 
-@pytest.mark.parametrize("M,K,T", [(96, 700, 45), (2048, 600, 301), (4096, 300, 1000)])
+# One shape for each of the tiles: 32 x 32, 64 x 64 with eight and with four
+# waves, 64 x 128.
+TILES = [(96, 700, 45), (2048, 600, 301), (8225, 270, 333), (4096, 300, 1000)]
+
+
+@pytest.mark.parametrize("M,K,T", TILES)
 def test_zero_runs(hl, M, K, T):
-    """Rows and columns that start with (or are) zeros: their scale comes from
-    their largest element, also where that is far from 1."""
+    """Rows and columns that start with (or are) zeros, also far from 1."""
     print(f"split gemm zero runs M={M} K={K} T={T}", flush=True)
     w, x = _operands(M, K, T, 5)
     w[3, :K // 2] = 0.0
@@ -76,19 +80,54 @@ def test_zero_runs(hl, M, K, T):
     _check(w, x)
 
 
-@pytest.mark.parametrize("M,K,T", [(96, 700, 45), (2048, 600, 301), (4096, 300, 1000)])
-def test_out_of_split_range(hl, M, K, T):
-    """Elements more than 2^9 above the first ones of their row or column,
-    and rows below 2^-100: the tile's fp32 MFMAs."""
-    print(f"split gemm out of range M={M} K={K} T={T}", flush=True)
+@pytest.mark.parametrize("R", [2.0 ** 12, 2.0 ** 20, 2.0 ** 31, 2.0 ** 60, 2.0 ** 100])
+@pytest.mark.parametrize("M,K,T", TILES)
+def test_large_beside_small(hl, M, K, T, R):
+    """Elements R times the others of their row (column), first in every
+    64-k chunk, at k = 5 alone, or among any wave's first 16 k, whose partners
+    are zero or 1 / R: the small elements' products are the result."""
+    print(f"split gemm large beside small M={M} K={K} T={T} R=2^{np.log2(R):.0f}", flush=True)
+    for every, partner in ((64, 0.0), (K, 0.0), (64, 1.0 / R), (32, 0.0)):
+        at = torch.arange(5 if every == K else 0, K, every, device="cuda")
+        for large_in_w in (True, False):
+            w, x = _operands(M, K, T, 9)
+            a, b = (w, x.t()) if large_in_w else (x.t(), w)
+            a[:, at] *= R
+            b[:, at] *= partner
+            _check(w, x)
+
+
+@pytest.mark.parametrize("M,K,T", TILES)
+def test_far_from_the_first(hl, M, K, T):
+    """Single elements far above the first ones of their row or column, and a
+    row far below the others."""
+    print(f"split gemm far from the first M={M} K={K} T={T}", flush=True)
     w, x = _operands(M, K, T, 6)
     w[40, K - 1] = 1e9
     x[K - 2, T - 3] = -3e12
     w[65] *= 1e-33
+    _check(w, x)
+
+
+@pytest.mark.parametrize("M,K,T", TILES)
+def test_small_parts(hl, M, K, T):
+    """Rows whose second and third bf16 parts are bf16 subnormals (held, and
+    multiplied as they are), and rows with bits below those, which send their
+    tiles to fp32 MFMAs; products down to 2^-140."""
+    print(f"split gemm small parts M={M} K={K} T={T}", flush=True)
+    w, x = _operands(M, K, T, 10)
+    w[4] = 2.0 ** -115 * (1.0 + 2.0 ** -16)
+    w[20, ::2] = 2.0 ** -109 * (1.0 + 2.0 ** -9 + 2.0 ** -17)
+    w[20, 1::2] = 0.0
+    _check(w, x)
+    w[36] *= 2.0 ** -120
+    w[68, :] = 0.0
+    w[68, K - 1] = 2.0 ** -140
+    x[:, 3] *= 2.0 ** 90
     _check(w, x, fp32=True)
 
 
-@pytest.mark.parametrize("M,K,T", [(96, 700, 45), (2048, 600, 301), (4096, 300, 1000)])
+@pytest.mark.parametrize("M,K,T", TILES)
 def test_inf_nan(hl, M, K, T):
     print(f"split gemm inf / nan M={M} K={K} T={T}", flush=True)
     w, x = _operands(M, K, T, 7)
