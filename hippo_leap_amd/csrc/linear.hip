@@ -309,13 +309,16 @@ __global__ __launch_bounds__(64 * KW, WM * WN == 8 ? 1 : 2) void linear_split_ke
   // Tile row r: its matrix and its row there behind m0.
   auto wbase = [&](int r) { return PAIR && (r & 16) ? wt2 : wt; };
   auto wrow = [&](int r) { return min(PAIR ? 16 * (r >> 5) + (r & 15) : r, mlast); };
-  uint32_t woff[NL];
+  // Offsets inside a tile: 32 bits hold those of all but the longest rows,
+  // which get the smallest tile (linear_plan).
+  typedef std::conditional_t<WM * WN == 1, size_t, uint32_t> Off;
+  Off woff[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int r = RPL * i + lrow;
-    woff[i] = (uint32_t)wrow(r) * (uint32_t)K + 4u * (uint32_t)(lp ^ (r & (C16 - 1)));
+    woff[i] = (Off)wrow(r) * (Off)K + (Off)(4 * (lp ^ (r & (C16 - 1))));
   }
-  const uint32_t xoff = (uint32_t)(8 * hh) * (uint32_t)T + (uint32_t)col0;
+  const Off xoff = (Off)(8 * hh) * (Off)T + (Off)col0;
   const int nfull = K / CK;
   const int nmine = wave < nfull ? (nfull - wave + KW - 1) / KW : 0;  // full chunks of this wave
   const bool tail = K % CK != 0 && wave == nfull % KW;                 // the last, partial chunk
@@ -641,6 +644,8 @@ LinearPlan linear_plan(const LinearCall& c) {
   for (int v = 0; v < (int)(sizeof(kSplit) / sizeof(kSplit[0])); ++v) {
     const SplitVariant& s = kSplit[v];
     if (c.T < s.bn / 32) continue;  // a lane holds bn / 32 columns
+    // Offsets of 32 bits inside a tile: 64 rows of K and 9 of T.
+    if (v > 0 && (c.K > (1 << 26) || c.T > (1 << 28))) continue;
     const int bm = c.pair ? s.bm / 2 : s.bm;
     long long tm[3] = {0, 0, 0};
     for (int i = 0; i < (c.pair ? 1 : c.nmat); ++i) tm[i] = ((long long)c.rows[i] + bm - 1) / bm;

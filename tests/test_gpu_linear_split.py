@@ -127,6 +127,24 @@ def test_small_parts(hl, M, K, T):
     _check(w, x, fp32=True)
 
 
+def test_longest_rows(hl):
+    """Rows so long that an element's offset inside a tile needs more than 32
+    bits (138.6 million columns: row 31 starts behind 2^32)."""
+    from hippo_leap_amd import attention as A
+    M, K, T = 32, 138_600_000, 2
+    print(f"split gemm longest rows M={M} K={K} T={T}", flush=True)
+    w = torch.empty(M, K, device="cuda")
+    for r in range(M):
+        w[r].fill_(float(r + 1))
+    x = torch.zeros(K, T, device="cuda")
+    x[::100_003] = torch.tensor([1.0, 3.0], device="cuda")
+    x[K - 1] = torch.tensor([2.0, 5.0], device="cuda")
+    y = torch.empty(M, T, device="cuda")
+    A.gpu_linear_col(y, x, w, K, M, T)
+    want = torch.arange(1, M + 1, device="cuda", dtype=torch.float64)[:, None] * x.double().sum(0)
+    assert torch.equal(y.double(), want)
+
+
 @pytest.mark.parametrize("M,K,T", TILES)
 def test_inf_nan(hl, M, K, T):
     print(f"split gemm inf / nan M={M} K={K} T={T}", flush=True)
