@@ -220,7 +220,7 @@ static bool qkv_launch(float* q, float* k, float* v, const float* x, const hl_la
 // workgroup of it reads.  A one-column norm is a launch of one workgroup that
 // nothing overlaps (4.5 us); the fold costs its GEMV about 1 us.  Llama-3.2-1B
 // shapes in Q4_K at 2K columns: 637 us a token with the fold in gate/up only,
-// 612 with it in Q/K/V and the head too.
+// 612 with it in Q/K/V (and the head) too.
 struct DecodeFlow {
   const hl_model_desc* m;
   float *x, *xn, *t0, *t1, *t2;
@@ -307,22 +307,12 @@ struct DecodeFlow {
     return HL_OK;
   }
 
-  // Final residual and norm, output projection, greedy token.
+  // Final residual and norm, output projection, greedy token.  Not folded:
+  // the step leaves the residual stream in x and its final norm in x_norm
+  // (4 us of the 612 above).
   int head(float* logits, int32_t* next) {
-    const void* const ws[1] = {m->output};
-    float* const ys[1] = {logits};
-    const size_t nb = (size_t)m->n_emb * 4, lb = (size_t)m->n_vocab * 4;
-    const auto clear = [&](const void* p, size_t bytes) { return !overlaps(logits, lb, p, bytes); };
-    // logits may lie in the scratch that the unfolded launches are done with
-    if (apart && m->output_type != 0 && clear(S, nb) && clear(T, nb) && clear(res, nb) &&
-        clear(m->output, (size_t)quant_row_bytes(m->output_type, m->n_emb) * m->n_vocab) &&
-        folded(linear_quant_norm_launch(1, ws, ys, &m->n_vocab, m->output_type, m->n_emb, T, S, res, m->output_norm,
-                                        m->rms_eps, (hipStream_t)stream))) {
-      if (hipGetLastError() != hipSuccess) return set_error(HL_EHIP, "fused norm output projection launch failed");
-    } else {
-      HL_TRY(norm(m->output_norm));
-      HL_TRY(linear_t(logits, xn, m->output, m->output_type, m->n_emb, m->n_vocab, 1, stream));
-    }
+    HL_TRY(norm(m->output_norm));
+    HL_TRY(linear_t(logits, xn, m->output, m->output_type, m->n_emb, m->n_vocab, 1, stream));
     return hl_argmax_async(logits, m->n_vocab, next, stream);
   }
 };

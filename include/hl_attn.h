@@ -588,9 +588,11 @@ typedef struct {
  * per layer Q/K/V projections (one launch when the three weights share a
  * quantized type, as K/V pairs and gate/up pairs are), qk-norm, RoPE,
  * K/V store, attention, O projection, residual + ffn norm, gate/up,
- * SiLU * up (the residual and norm inside the gate/up launch when that runs
- * Q4_K on the matrix cores), down, residual + next layer's norm; final norm, output
- * projection, argmax.  Sets the process-wide RoPE table
+ * SiLU * up, down, residual + next layer's norm (a residual and norm inside
+ * the Q/K/V or gate/up launch behind it where that runs on the matrix cores:
+ * one of Q4_K, Q5_K, Q6_K, Q8_0 for all its matrices); final norm, output
+ * projection, argmax.  Afterwards x holds the residual stream and x_norm its
+ * final norm; what tmp0 .. tmp2 hold is undefined.  Sets the process-wide RoPE table
  * (hl_set_rope_theta) on every call: steps of models with different RoPE
  * parameters must not run concurrently (the reference's theta table is
  * module-global too).                                                     */
@@ -682,7 +684,8 @@ int hl_forward_prefill(const hl_model_desc* model, hl_kv_cache_desc* cache,
  * cache->cur_len += 1.  fp16/bf16/fp8 caches run each layer's qk-norm,
  * RoPE, cache write and attention as one launch (hl_decode_step); fp32
  * caches run the reference's sequence.  Weights fp32 or any GGUF type of
- * hl_gpu_linear_col_quant.  "KV cache full" (HL_ECAPACITY) when cur_len ==
+ * hl_gpu_linear_col_quant.  x and x_norm of the scratch hold the residual
+ * stream and its final norm afterwards.  "KV cache full" (HL_ECAPACITY) when cur_len ==
  * max_len.  Nothing allocates or waits for the stream.                    */
 int hl_forward_decode(const hl_model_desc* model, hl_kv_cache_desc* cache,
                       const hl_forward_scratch* scratch, const int32_t* token_dev,

@@ -183,10 +183,19 @@ def test_forward_decode_token_norm_folded_into_gate_up(hl, orc, n_emb, n_ff):
         m.tokens[0] = tok
 
 
-# Residual + norm folded into the Q/K/V launch (3072 x 2048) and the output
-# projection (2100 x 2048): one type each, scratch wide enough for q behind
-# the residual (n_ff >= 2 n_emb); at 4032 it is not and only the head folds.
-# logits in tmp0 (allowed, the unfolded head is done with it) must not fold.
+# Residual + norm folded into the Q/K/V launch (3072 x 2048), of one type;
+# scratch wide enough for q behind the residual (n_ff >= 2 n_emb), at 4032 it
+# is not.  The head does not fold: it leaves the residual stream in x and the
+# final norm in x_norm.  logits may lie in tmp0, which it is done with.
+def _check_hidden(bufs, cfg, ref, logits):
+    """x and x_norm after a step: the residual stream (its norm times the
+    output weights gives the logits) and its final norm."""
+    x, xn = (b[:cfg["n_emb"]].cpu().numpy().astype(np.float64) for b in bufs[:2])
+    want = x / np.sqrt((x * x).mean() + cfg["rms_eps"]) * ref["output_norm"]
+    assert rel_err(xn, want) < TOL_F32
+    assert rel_err(logits, ref["output"].reshape(-1, len(xn)).astype(np.float64) @ xn) < TOL_F32
+
+
 @pytest.mark.parametrize("qtype,n_ff,logits_in_tmp0", [(8, 4096, False), (12, 4352, False), (13, 4096, False),
                                                        (14, 4096, False), (8, 4032, False), (8, 4096, True)])
 def test_forward_decode_norm_folded_into_qkv_and_head(hl, orc, qtype, n_ff, logits_in_tmp0):
@@ -207,10 +216,12 @@ def test_forward_decode_norm_folded_into_qkv_and_head(hl, orc, qtype, n_ff, logi
         ref_logits = _oracle_step(orc, cfg, ref, tok, pos)
         assert rel_err(logits, ref_logits) < TOL_F32, f"step {pos}"
         assert nxt == orc.argmax(logits)
+        _check_hidden(m.fbufs, cfg, ref, logits)
         if not logits_in_tmp0:  # the descriptor's own caches, same step
             m.step(pos)
             torch.cuda.synchronize()
             assert rel_err(m.logits.cpu().numpy(), ref_logits) < TOL_F32, f"step {pos}"
+            _check_hidden(m.bufs, cfg, ref, m.logits.cpu().numpy())
         tok = nxt
 
 
