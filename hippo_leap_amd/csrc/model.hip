@@ -543,12 +543,13 @@ static int check_workspace(const hl_forward_scratch* s, size_t need) {
 
 // One launch of the fp32 projections that share x (LinearCall); a single
 // column goes through the GEMVs, a residual (onto y[0] itself) by way of tmp.
-static int prefill_linear(const LinearCall& c, void* stream, float* tmp = nullptr) {
-  // The refusals of hl_gpu_linear_col, tmp included.
+// tmp and tmp2: scratch of the launches that this one replaces.
+static int prefill_linear(const LinearCall& c, void* stream, float* tmp = nullptr, float* tmp2 = nullptr) {
+  // The refusals of hl_gpu_linear_col, the scratch included.
   const size_t xb = (size_t)c.K * c.T * 4;
   for (int i = 0; i < c.nmat; ++i) {
     const size_t yb = (size_t)c.rows[i] * c.T * 4;
-    for (const float* y : {c.pair ? c.y[0] : c.y[i], tmp})
+    for (const float* y : {c.pair ? c.y[0] : c.y[i], tmp, tmp2})
       if (y && (overlaps(y, yb, c.x, xb) || overlaps(y, yb, c.w[i], (size_t)c.rows[i] * c.K * 4)))
         return set_error(HL_EINVAL, "linear_col: dst overlaps x or w");
   }
@@ -600,7 +601,7 @@ int hl_forward_prefill(const hl_model_desc* m, hl_kv_cache_desc* c, const hl_for
     HL_TRY(hl_gpu_rmsnorm_cols(xn, x, L.ffn_norm, E, T, eps, stream));
     const float *wg = (const float*)L.w_gate, *wu = (const float*)L.w_up;
     if (T > 1) {
-      HL_TRY(prefill_linear({2, {wg, wu}, {t2}, {m->n_ff, m->n_ff}, xn, nullptr, true, E, T}, stream));
+      HL_TRY(prefill_linear({2, {wg, wu}, {t2}, {m->n_ff, m->n_ff}, xn, nullptr, true, E, T}, stream, t0, t1));
     } else {
       HL_TRY(prefill_linear({2, {wg, wu}, {t0, t1}, {m->n_ff, m->n_ff}, xn, nullptr, false, E, T}, stream));
       HL_TRY(hl_gpu_silu_mul(t2, t0, t1, m->n_ff, stream));

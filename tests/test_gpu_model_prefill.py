@@ -288,6 +288,26 @@ def test_prefill_refuses_overlapping_scratch(hl, orc, T, buf, onto):
     torch.cuda.synchronize()
 
 
+# tmp0 (tmp1) of n_ff columns reaching into x_norm behind the n_emb and
+# n_head * head_dim columns that the projections before gate / up write there.
+@pytest.mark.parametrize("T", [1, 5])
+@pytest.mark.parametrize("buf", ["tmp0", "tmp1"])
+def test_prefill_refuses_gate_and_up_reaching_into_x_norm(hl, orc, T, buf):
+    from hippo_leap_amd import _lib
+    from hippo_leap_amd.model import DenseModel
+    print(f"prefill {buf} reaching into x_norm T={T}", flush=True)
+    cfg = dict(CFG, n_ff=4 * max(CFG["n_emb"], CFG["n_head"] * CFG["head_dim"]))
+    dev, _ = _build(orc, cfg, {}, False, 7)
+    m = DenseModel(torch, cfg, dev["tok_emb"], dev["output_norm"], dev["output"], 0, dev["layers"], max_tokens=8)
+    n = cfg["n_ff"] // 4 * T
+    both = torch.zeros(8 * cfg["n_ff"], device="cuda")
+    setattr(m.fscratch, buf, both.data_ptr())
+    m.fscratch.x_norm = both[n:].data_ptr()
+    with pytest.raises(_lib.HLError, match="overlap"):
+        m.prefill(list(range(T)))
+    torch.cuda.synchronize()
+
+
 def test_decode_refuses_overlapping_norm_buffer(hl):
     """x_norm on x: the residual norm refuses it, also at a size whose Q/K/V
     and gate/up launches could take the norm in."""
