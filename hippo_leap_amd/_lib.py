@@ -18,6 +18,9 @@ HL_KV_COLMAJOR, HL_KV_TILED32, HL_KV_PAGED32 = 0, 1, 2
 HL_GGML_F16, HL_GGML_Q5_0, HL_GGML_Q5_1, HL_GGML_Q8_0 = 1, 6, 7, 8
 HL_GGML_Q2_K, HL_GGML_Q3_K, HL_GGML_Q4_K, HL_GGML_Q5_K, HL_GGML_Q6_K = 10, 11, 12, 13, 14
 HL_GGML_IQ4_NL = 20
+# Kernels of the linear layers (hl_linear_launches).
+(HL_LK_GEMV, HL_LK_SPLIT_32X32, HL_LK_SPLIT_64X64_W8, HL_LK_SPLIT_64X64_W4, HL_LK_SPLIT_64X128, HL_LK_QUANT,
+ HL_LK_Q4K_MFMA, HL_LK_Q4K_MFMA_NORM, HL_LK_I8, HL_LK_I8_NORM, HL_LK_KINDS) = range(11)
 
 c_int, c_float, c_void_p, c_size_t, c_longlong = (
     ctypes.c_int, ctypes.c_float, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_longlong)
@@ -118,6 +121,7 @@ class PrefillArgs(ctypes.Structure):
 SIGNATURES = {
     "hl_last_error": (ctypes.c_char_p, []),
     "hl_abi_version": (c_int, []),
+    "hl_linear_launches": (ctypes.c_longlong, [c_int]),
     "hl_device_info_get": (c_int, [ctypes.POINTER(DeviceInfo)]),
     "hl_rope_theta_table": (c_int, [ctypes.POINTER(c_float), c_int, c_float]),
     "hl_set_rope_theta": (c_int, [c_int, c_float]),

@@ -162,6 +162,9 @@ size_t prefill_f32_split_bytes(int n_head_kv, int head_dim, int seq_len);
 hipError_t prefill_mfma_launch(const PrefillLaunch& p, hipStream_t stream);
 int prefill_mfma_tpad(int seq_len);
 
+// Notes a launch of a linear layer's kernel (HL_LK_*) for hl_linear_launches.
+void count_linear(int kernel);
+
 // ---- fp32 linear layer (linear.hip) ----------------------------------------
 // Y[M, T] = W[M, K] . X[K, T]: GEMV for T == 1, GEMM on split operands otherwise.
 // One GEMM launch over up to three matrices and the same X (T >= 2): y[i] =

@@ -672,6 +672,10 @@ static void launch_split(const SplitArgs& a, bool pair, hipStream_t stream) {
   else hipLaunchKernelGGL((linear_split_kernel<WM, WN, KW, CK, XD, false>), grid, block, 0, stream, a);
 }
 
+static thread_local long long g_linear_launches[HL_LK_KINDS];
+
+void count_linear(int kernel) { ++g_linear_launches[kernel]; }
+
 hipError_t linear_cols_launch(const LinearCall& c, hipStream_t stream) {
   const LinearPlan p = linear_plan(c);
   if (p.tiles_m == 0) return hipErrorInvalidValue;
@@ -694,12 +698,14 @@ hipError_t linear_cols_launch(const LinearCall& c, hipStream_t stream) {
   else if (p.variant == 1) launch_split<2, 2, 8, 32, 2>(a, c.pair, stream);
   else if (p.variant == 2) launch_split<2, 2, 4, 32, 2>(a, c.pair, stream);
   else launch_split<2, 4, 4, 32, 2>(a, c.pair, stream);
+  count_linear(HL_LK_SPLIT_32X32 + p.variant);
   return hipGetLastError();
 }
 
 hipError_t linear_col_launch(float* y, const float* x, const float* w, int K, int M, int T,
                              hipStream_t stream) {
   if (T > 1) return linear_cols_launch(LinearCall{1, {w}, {y}, {M}, x, nullptr, false, K, T}, stream);
+  count_linear(HL_LK_GEMV);
   const bool vec = K % 4 == 0 && aligned16(w) && aligned16(x);
   const int wpr = M >= 2048 ? 1 : 4;
   const dim3 grid((M + 4 / wpr - 1) / (4 / wpr)), block(256);
@@ -714,3 +720,7 @@ hipError_t linear_col_launch(float* y, const float* x, const float* w, int K, in
 }
 
 }  // namespace hl
+
+extern "C" long long hl_linear_launches(int kernel) {
+  return kernel >= 0 && kernel < HL_LK_KINDS ? hl::g_linear_launches[kernel] : 0;
+}

@@ -1115,8 +1115,9 @@ __global__ __launch_bounds__(1024) void q4k_mfma_kernel(const uint8_t* __restric
   }
 }
 
-// What the int8 kernel does not take (K < 2048 or > 16384, rows not on 16
-// bytes).  The MFMA kernel pays for its x prologue (~2 us of latency before the
+// What the int8 kernel does not take: K < 2048 or > 16384, rows not on 16
+// bytes, and row counts that leave its last round of workgroups mostly empty
+// (8193 x 4096; pairs of 8195 x 2048).  The MFMA kernel pays for its x prologue (~2 us of latency before the
 // first product) on matrices of 2^25 weights and more: 14336 x 4096 10.8 us
 // against 15.7, 4096 x 14336 14.2 against 17.0, but 4096 x 4096 8.3 against
 // 6.6 (kernel durations).  A fused pair streams both matrices behind one x
@@ -1166,6 +1167,7 @@ bool launch_q4k_mfma(const uint8_t* w, const float* x, float* y, int M, int K, h
   }
   hipLaunchKernelGGL((q4k_mfma_kernel<PAIR, NORM>), dim3((M + rows - 1) / rows), dim3(64 * nw), shm, stream, w,
                      x, y, M, K, w2, y2, rows, res, nrm, xsum, eps);
+  count_linear(NORM ? HL_LK_Q4K_MFMA_NORM : HL_LK_Q4K_MFMA);
   return true;
 }
 
@@ -1177,6 +1179,7 @@ void launch_direct(const uint8_t* w, const float* x, float* y, int M, int K, hip
   const int grid = (groups + 4 / KS - 1) / (4 / KS);
   hipLaunchKernelGGL((quant_direct_kernel<QT, R, KS, PAIR>), dim3(grid), dim3(256), 0, stream, w, x, y,
                      M, K, w2, y2, w3, y3, M2);
+  count_linear(HL_LK_QUANT);
 }
 
 // The int8 matrix-core kernel (linear_quant_i8.hip) has 1.3-3 us more of
@@ -1283,6 +1286,7 @@ bool launch_pair_qt(const uint8_t* w, const uint8_t* w2, const float* x, float* 
 template <int QT, int WPR>
 void launch_q(const uint8_t* w, const float* x, float* y, int M, int K, bool aligned, bool v4,
               hipStream_t stream) {
+  count_linear(HL_LK_QUANT);
   const dim3 grid((M + 4 / WPR - 1) / (4 / WPR)), block(256);
   if (aligned) {
     if (v4) hipLaunchKernelGGL((quant_gemv_kernel<QT, WPR, true, true>), grid, block, 0, stream, w, x, y, M, K);
@@ -1475,9 +1479,13 @@ hipError_t linear_quant_launch(float* y, const float* x, const void* w, int K, i
   const uint8_t* wb = (const uint8_t*)w;
   switch (qtype) {
     case HL_GGML_F16:
-      if (K % 32 == 0) launch_qt<1>(wb, x, y, M, K, stream);
-      else hipLaunchKernelGGL(f16_gemv_any_kernel, dim3((M + 3) / 4), dim3(256), 0, stream,
-                              (const uint16_t*)w, x, y, M, K);
+      if (K % 32 == 0) {
+        launch_qt<1>(wb, x, y, M, K, stream);
+      } else {
+        hipLaunchKernelGGL(f16_gemv_any_kernel, dim3((M + 3) / 4), dim3(256), 0, stream, (const uint16_t*)w, x, y, M,
+                           K);
+        count_linear(HL_LK_QUANT);
+      }
       break;
     case HL_GGML_Q5_0: launch_qt<6>(wb, x, y, M, K, stream); break;
     case HL_GGML_Q5_1: launch_qt<7>(wb, x, y, M, K, stream); break;

@@ -480,6 +480,7 @@ bool launch(QmArgs a, int nsb, hipStream_t stream) {
   if (!NORM && (float)a.ngroups < full * (float)rounds * (float)slots) return false;
   const int grid = std::min(a.ngroups, slots);
   hipLaunchKernelGGL((quant_i8_kernel<QT, MAX, PAIR, NORM, XQ>), dim3(grid), dim3(64 * nsb), shm, stream, a);
+  count_linear(NORM ? HL_LK_I8_NORM : HL_LK_I8);
   return true;
 }
 

@@ -250,6 +250,25 @@ int hl_gpu_linear_col_quant(float* dst, const float* x, const void* w_quant,
                             int w_cols, int w_rows, int quant_type,
                             void* stream);
 
+/* The kernels that the linear layers choose between, and how many launches of
+ * each the calling thread has made (every device and stream, the model calls'
+ * included; 0 for another number): for tests and profiling, which kernel a
+ * shape takes.  Extends the reference.                                      */
+enum {
+  HL_LK_GEMV = 0,                 /* fp32, one column                        */
+  HL_LK_SPLIT_32X32 = 1,          /* fp32 columns: tile and waves            */
+  HL_LK_SPLIT_64X64_W8 = 2,
+  HL_LK_SPLIT_64X64_W4 = 3,
+  HL_LK_SPLIT_64X128 = 4,
+  HL_LK_QUANT = 5,                /* quantized, on the vector ALUs           */
+  HL_LK_Q4K_MFMA = 6,             /* Q4_K on fp16 matrix cores               */
+  HL_LK_Q4K_MFMA_NORM = 7,        /* ... with the residual and norm in it    */
+  HL_LK_I8 = 8,                   /* quantized on int8 matrix cores          */
+  HL_LK_I8_NORM = 9,
+  HL_LK_KINDS = 10
+};
+long long hl_linear_launches(int kernel);
+
 /* gpuRmsnormCols (naive.nim:2834-2843): dst[r, t] = x[r, t] *
  * (1/sqrtf(sum_r x[r, t]^2 / dim + eps)) * weight[r] over the col-major
  * fp32 [dim, seqLen] (the norm in front of the Q/K/V projections and the

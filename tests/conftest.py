@@ -34,6 +34,15 @@ def _library_stale(lib_path: str) -> bool:
     return any(os.path.getmtime(s) > built for s in sources if os.path.isfile(s))
 
 
+@pytest.fixture
+def launches(hl):
+    """launches(kernel): launches of that linear layer kernel (HL_LK_*) since
+    the test began, so that a test can say which kernel its shapes take."""
+    from hippo_leap_amd import _lib
+    start = [hl.hl_linear_launches(k) for k in range(_lib.HL_LK_KINDS)]
+    return lambda k: hl.hl_linear_launches(k) - start[k]
+
+
 @pytest.fixture(scope="session")
 def orc():
     import oracle

@@ -15,6 +15,8 @@ import numpy as np
 import pytest
 import torch
 
+from hippo_leap_amd import _lib
+
 pytestmark = pytest.mark.gpu
 
 
@@ -46,23 +48,27 @@ def _operands(M, K, T, seed, offset=0):
     return w, x
 
 
-SHAPES = [(1, 1, 2), (33, 15, 2), (31, 16, 3), (32, 17, 31), (65, 63, 32), (64, 64, 33), (130, 65, 63), (70, 511, 65),
-          (96, 513, 127), (5, 1003, 129), (257, 4099, 7),             # 32 x 32 tiles
-          (2048, 512, 301), (2081, 545, 257), (2111, 97, 303),        # 64 x 64
-          (8192, 256, 301), (8225, 129, 333),                         # 64 x 64, four waves
-          (4096, 256, 1000), (4133, 161, 1027), (3001, 191, 2049)]    # 64 x 128
+# M, K, T and the tile that takes them.
+SHAPES = [(*s, kind) for kind, shapes in {
+    _lib.HL_LK_SPLIT_32X32: [(1, 1, 2), (33, 15, 2), (31, 16, 3), (32, 17, 31), (65, 63, 32), (64, 64, 33),
+                             (130, 65, 63), (70, 511, 65), (96, 513, 127), (5, 1003, 129), (257, 4099, 7)],
+    _lib.HL_LK_SPLIT_64X64_W8: [(2048, 512, 301), (2081, 545, 257), (2111, 97, 303)],
+    _lib.HL_LK_SPLIT_64X64_W4: [(8192, 256, 301), (8225, 129, 333), (4096, 256, 1000), (4133, 161, 1027),
+                                (3001, 191, 2049)],
+    _lib.HL_LK_SPLIT_64X128: [(2048, 1024, 1000), (2033, 1003, 1021), (2001, 1031, 1024), (1985, 1489, 1009)],
+}.items() for s in shapes]
 
 
-@pytest.mark.parametrize("M,K,T", SHAPES)
-def test_edges(hl, M, K, T):
+@pytest.mark.parametrize("M,K,T,kind", SHAPES)
+def test_edges(hl, launches, M, K, T, kind):
     print(f"split gemm M={M} K={K} T={T}", flush=True)
     for offset in (0, 1):  # addresses on 16 and on 4 bytes
         _check(*_operands(M, K, T, 17 * M + K + T, offset))
+    assert launches(kind) == 2
 
 
-# One shape for each of the tiles: 32 x 32, 64 x 64 with eight and with four
-# waves, 64 x 128.
-TILES = [(96, 700, 45), (2048, 600, 301), (8225, 270, 333), (4096, 300, 1000)]
+# One shape for each tile (two for the 64 x 64 one of four waves).
+TILES = [(96, 700, 45), (2048, 600, 301), (8225, 270, 333), (4096, 300, 1000), (2033, 1003, 1021)]
 
 
 @pytest.mark.parametrize("M,K,T", TILES)

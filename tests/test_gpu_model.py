@@ -13,6 +13,7 @@ import pytest
 import torch
 
 from gguf_pack import random_rows
+from hippo_leap_amd import _lib
 from util import TOL_F32, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -159,11 +160,13 @@ def test_forward_decode_token_wide_fused_projections(hl, orc, types):
 CFG_FFN = dict(CFG, n_emb=2048, n_head=32, n_head_kv=8, n_ff=16384)
 
 
-# The fold at other widths: K = 4096 (two 8-block groups, eight waves, the
-# Llama-3-8B width), 8192 (four groups, sixteen waves) and 2560 (ten blocks:
-# a partial second group, threads past K/8 load zeros and write no sum).
-@pytest.mark.parametrize("n_emb,n_ff", [(2048, 16384), (2048, 8192), (4096, 4096), (8192, 2048), (2560, 6656)])
-def test_forward_decode_token_norm_folded_into_gate_up(hl, orc, n_emb, n_ff):
+# The fold at other widths: on the int8 kernel K = 4096 (one step of sixteen
+# waves, the Llama-3-8B width), 8192 (two steps) and 2560 (ten waves); on the
+# fp16 kernel K = 1792 (seven blocks of a group of eight: threads past K/8 load
+# zeros and write no sum).
+@pytest.mark.parametrize("n_emb,n_ff", [(2048, 16384), (2048, 8192), (4096, 4096), (8192, 2048), (2560, 6656),
+                                        (1792, 9472)])
+def test_forward_decode_token_norm_folded_into_gate_up(hl, orc, launches, n_emb, n_ff):
     from hippo_leap_amd.model import DenseDecoder
     types = {"wq": 12, "wk": 12, "wv": 12, "wo": 12, "w_gate": 12, "w_up": 12, "w_down": 12}
     print(f"decode model: norm folded into the Q4_K gate/up, n_emb {n_emb} n_ff {n_ff}", flush=True)
@@ -181,6 +184,32 @@ def test_forward_decode_token_norm_folded_into_gate_up(hl, orc, n_emb, n_ff):
         assert rel_err(logits, ref_logits) < TOL_F32, f"step {pos}"
         tok = int(m.tokens[1].item())
         m.tokens[0] = tok
+    fp16 = n_emb == 1792
+    assert launches(_lib.HL_LK_Q4K_MFMA_NORM) == (3 * cfg["n_layer"] if fp16 else 0)
+    assert (launches(_lib.HL_LK_I8_NORM) >= 3 * cfg["n_layer"]) == (not fp16)
+
+
+# The folds of the Q/K/V and gate/up launches at the Llama-3-8B width: K = 4096
+# is one step of sixteen waves, for Q8_0 two steps of eight.
+@pytest.mark.parametrize("qtype", [8, 12, 13, 14])
+def test_forward_decode_folds_at_width_4096(hl, orc, launches, qtype):
+    from hippo_leap_amd.model import DenseModel
+    print(f"decode model: folds at width 4096, type {qtype}", flush=True)
+    cfg = dict(CFG_WIDE, n_emb=4096, n_ff=6144)
+    types = {n: qtype for n in ("wq", "wk", "wv", "wo", "w_gate", "w_up", "w_down", "output")}
+    dev, ref = _build(orc, cfg, types, False, 211)
+    m = DenseModel(torch, cfg, dev["tok_emb"], dev["output_norm"], dev["output"], dev["output_type"], dev["layers"])
+    tok = 9
+    for pos in range(2):
+        m.tokens[0] = tok
+        m.decode()
+        torch.cuda.synchronize()
+        logits = m.logits.cpu().numpy()
+        assert rel_err(logits, _oracle_step(orc, cfg, ref, tok, pos)) < TOL_F32, f"step {pos}"
+        _check_hidden(m.fbufs, cfg, ref, logits)
+        tok = int(m.tokens[1].item())
+    # gate/up of both layers, Q/K/V of the second
+    assert launches(_lib.HL_LK_I8_NORM) == 2 * (2 * cfg["n_layer"] - 1)
 
 
 # Residual + norm folded into the Q/K/V launch (3072 x 2048), of one type;

@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from gguf_pack import random_rows
+from hippo_leap_amd import _lib
 
 pytestmark = pytest.mark.gpu
 BOUND = 1.2e-5
@@ -46,11 +47,22 @@ def _close(got, ref):
 
 SHAPES = [(20471, 2048), (20200, 2304), (16375, 3840), (12279, 4096), (12200, 4352), (8187, 4864), (4087, 8704),
           (4081, 14336), (4090, 16384)]
+# Q6_K takes multiples of eight superblocks and 40 million weights, Q8_0 below
+# K = 4096 1.5 2^25 weights; the others of these run on the vector ALUs.
+SHAPES_OF = {Q4_K: SHAPES, Q5_K: SHAPES,
+             Q6_K: SHAPES + [(8180, 6144), (8187, 8192)],
+             Q8_0: SHAPES + [(24583, 2048), (23000, 2304), (27999, 2304)]}
+ON_ALUS = [(Q6_K, M, K) for M, K in SHAPES if K in (2304, 3840, 4352, 4864, 8704)] + [
+    (Q8_0, 20471, 2048), (Q8_0, 20200, 2304), (Q8_0, 12283, 2048), (Q6_K, 6100, 4352)]
 
 
-@pytest.mark.parametrize("qtype", [Q4_K, Q5_K, Q6_K, Q8_0])
-@pytest.mark.parametrize("M,K", SHAPES)
-def test_one(hl, orc, qtype, M, K):
+def _took(launches, qtype, M, K, n):
+    alus = (qtype, M, K) in ON_ALUS
+    assert (launches(_lib.HL_LK_QUANT), launches(_lib.HL_LK_I8)) == ((n, 0) if alus else (0, n))
+
+
+@pytest.mark.parametrize("qtype,M,K", [(q, *s) for q, shapes in SHAPES_OF.items() for s in shapes])
+def test_one(hl, orc, launches, qtype, M, K):
     from hippo_leap_amd import attention as A
     print(f"int8 gemv type {qtype} M={M} K={K}", flush=True)
     w, times = _weights(orc, qtype, M, K, M + qtype)
@@ -62,11 +74,15 @@ def test_one(hl, orc, qtype, M, K):
     again = torch.empty(M, device="cuda")
     A.gpu_linear_col_quant(again, x, w, K, M, qtype)
     assert torch.equal(again, y[:M])
+    _took(launches, qtype, M, K, 2)
 
 
-@pytest.mark.parametrize("qtype", [Q4_K, Q5_K, Q6_K, Q8_0])
-@pytest.mark.parametrize("M,K", [(12283, 2048), (6139, 4096), (6100, 4352), (4093, 8192), (4083, 14336)])
-def test_pairs(hl, orc, qtype, M, K):
+PAIRS = [(12283, 2048), (6139, 4096), (6100, 4352), (4093, 8192), (4083, 14336)]
+PAIRS_OF = {Q4_K: PAIRS, Q5_K: PAIRS, Q6_K: PAIRS + [(8190, 6144)], Q8_0: PAIRS + [(12300, 2048), (14331, 2304)]}
+
+
+@pytest.mark.parametrize("qtype,M,K", [(q, *s) for q, shapes in PAIRS_OF.items() for s in shapes])
+def test_pairs(hl, orc, launches, qtype, M, K):
     from hippo_leap_amd import attention as A
     print(f"int8 pair type {qtype} M={M} K={K}", flush=True)
     wa, ta = _weights(orc, qtype, M, K, M)
@@ -84,14 +100,16 @@ def test_pairs(hl, orc, qtype, M, K):
     A.gpu_fused_kv_linear_quant(k, v, x, wa, wb, K, M, qtype, qtype)
     _close(k, a)
     _close(v, b)
+    _took(launches, qtype, M, K, 2)
 
 
-@pytest.mark.parametrize("qtype", [Q4_K, Q6_K, Q8_0])
-def test_large_and_non_finite_x(hl, orc, qtype):
-    """x up to the fp32 range is held exactly; an inf or NaN in x makes every
-    row NaN (q x summed with its offset or min, as in fp32)."""
+@pytest.mark.parametrize("qtype,M", [(Q4_K, 20480), (Q5_K, 20480), (Q6_K, 20480), (Q8_0, 20480), (Q8_0, 24583)])
+def test_large_and_non_finite_x(hl, orc, launches, qtype, M):
+    """x up to the fp32 range is held to 2^-31 of its superblock's largest; an
+    inf or NaN in x makes every row NaN (q x summed with its offset or min, as
+    in fp32)."""
     from hippo_leap_amd import attention as A
-    M, K = 20480, 2048
+    K = 2048
     w, times = _weights(orc, qtype, M, K, 77)
     x = _x(K, 5) * 1e33
     y = torch.empty(M, device="cuda")
@@ -101,3 +119,5 @@ def test_large_and_non_finite_x(hl, orc, qtype):
         x[700] = bad
         A.gpu_linear_col_quant(y, x, w, K, M, qtype)
         assert bool(torch.isnan(y).all())
+    alus = (qtype, M) == (Q8_0, 20480)
+    assert launches(_lib.HL_LK_QUANT if alus else _lib.HL_LK_I8) == 3
