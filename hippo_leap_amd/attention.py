@@ -44,7 +44,11 @@ def dtype_code(t: torch.Tensor) -> int:
 # part of its time: pointers go to ctypes as plain integers (its argtypes make
 # the c_void_p), and the current stream's handle is read without building a
 # torch.cuda.Stream around it: gpu_add 7.0 -> 4.2 us, of which 3.3 are the
-# launch itself.
+# launch itself.  (The call that gives the handle is not in torch's documented
+# interface; without it the stream object is built.)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _p(t):
     """Device pointer of a tensor (or None)."""
     if t is None:
@@ -58,7 +62,9 @@ def _stream(stream=None):
     """Handle of a torch stream (default: the current device's current one)."""
     if stream is not None:
         return stream.cuda_stream
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 # ---------------------------------------------------------------------------

@@ -458,3 +458,18 @@ def test_bench_refuses_more_than_one_gpu():
     assert r.returncode == 2
     msg = json.loads(r.stdout.strip().splitlines()[-1])
     assert "one GPU" in msg["error"]
+
+
+def test_current_stream_without_the_raw_handle(monkeypatch):
+    """A torch without the call that gives the current stream's handle: the
+    wrappers take it from the stream object."""
+    from types import SimpleNamespace
+
+    from hippo_leap_amd import attention as A
+    monkeypatch.setattr(A, "_raw_stream", None)
+    monkeypatch.setattr(A.torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=1234))
+    assert A._stream() == 1234
+    monkeypatch.setattr(A, "_raw_stream", lambda device: 5678 + device)
+    monkeypatch.setattr(A.torch.cuda, "current_device", lambda: 1)
+    assert A._stream() == 5679
+    assert A._stream(SimpleNamespace(cuda_stream=9)) == 9
