@@ -245,7 +245,11 @@ enum {
  * kernel, naive.nim:1267-1323).  wCols must be a multiple of the block (32;
  * 256 for the K-quants; any for F16): HL_EINVAL with the reference's
  * row-size message otherwise.  Other types: HL_EUNSUPPORTED ("unsupported
- * quant type for GPU GEMV: <type>").  dst must not overlap x or w.        */
+ * quant type for GPU GEMV: <type>").  dst must not overlap x or w.  Q4_K,
+ * Q5_K, Q6_K and Q8_0 matrices of 2^25 weights and more (2^22 inside a decode
+ * step) run on the matrix cores, which hold x to 2^-31 of the largest of each
+ * 256 elements (the Q4_K shapes left to the fp16 cores: to 2^-22 of each
+ * element); an inf or a NaN in x makes every row NaN.                      */
 int hl_gpu_linear_col_quant(float* dst, const float* x, const void* w_quant,
                             int w_cols, int w_rows, int quant_type,
                             void* stream);

@@ -1,11 +1,11 @@
 """GPU parity: the fp32 linear layer (hl_gpu_linear_col, the drop-in for
 gpuLinearCol, backends/naive.nim:3519-3547) against the CPU oracle's
 restatement of tensor.nim's matmul (tensor.nim:63-81), on both kernels:
-the decode GEMV (seq_len == 1) and the fp32-MFMA GEMM (seq_len > 1), with
-and without 16-byte loads (K or T not a multiple of 4, misaligned inputs),
-ragged tiles, and at the Llama-3-8B projection shapes against an fp64
-matmul of the same inputs; the 128 x 128-tile GEMM also over wide exponent
-ranges and with inf / NaN operands.  Bar: 1e-4 relative (fp32)."""
+the decode GEMV (seq_len == 1, with and without 16-byte loads) and the GEMM
+on split operands (seq_len > 1), with K or T not a multiple of 4, misaligned
+inputs and ragged tiles, and at the Llama-3-8B projection shapes against an
+fp64 matmul of the same inputs; the GEMM also over wide exponent ranges and
+with inf / NaN operands.  Bar: 1e-4 relative (fp32)."""
 import numpy as np
 import pytest
 import torch
@@ -36,12 +36,12 @@ CASES = [
     (37, 130, 1, 0),      # K % 4 != 0: one float per lane
     (5, 3, 1, 0),         # tiny
     (300, 1000, 1, 1),    # misaligned x: scalar loads
-    (256, 512, 64, 0),    # GEMM, 64x64 tiles, exact
-    (200, 96, 7, 0),      # T % 4 != 0: scalar loads, ragged tile
+    (256, 512, 64, 0),    # GEMM, whole tiles
+    (200, 96, 7, 0),      # T % 4 != 0, ragged tile
     (130, 100, 33, 0),    # K not a multiple of 32 or 4, ragged M and T
     (64, 64, 2, 0),       # smallest prefill
     (96, 72, 40, 2),      # misaligned x
-    (2048, 40, 4096, 0),  # 128x128 tiles (>= 512 tiles), K tail inside one chunk
+    (2048, 40, 4096, 0),  # many tiles, K tail inside one chunk
 ]
 
 
@@ -91,8 +91,8 @@ def test_linear_col_linearity_and_repeat(hl, orc):
     assert torch.equal(ys[0], ys[3])
 
 
-def _tile128_operands(seed):
-    """2048 x 4096 outputs (512 tiles: the 128 x 128-tile GEMM), K = 256."""
+def _wide_operands(seed):
+    """2048 x 4096 outputs (64 x 64 tiles, several rounds of them), K = 256."""
     g = torch.Generator(device="cuda").manual_seed(seed)
     M, K, T = 2048, 256, 4096
     w = torch.rand(M, K, device="cuda", generator=g) * 2 - 1
@@ -105,7 +105,7 @@ def test_linear_col_gemm_wide_range(hl):
     every output within 1e-4 of its own row/column scale against a float64
     matmul."""
     from hippo_leap_amd import attention as A
-    M, K, T, w, x = _tile128_operands(41)
+    M, K, T, w, x = _wide_operands(41)
     rs = torch.logspace(-18, 18, M, device="cuda")
     cs = torch.logspace(-15, 15, T, device="cuda")
     w = w * rs[:, None]
@@ -124,7 +124,7 @@ def test_linear_col_gemm_inf_nan(hl):
     reference's fp32 products do; every other output matches a float64
     matmul."""
     from hippo_leap_amd import attention as A
-    M, K, T, w, x = _tile128_operands(42)
+    M, K, T, w, x = _wide_operands(42)
     x = x.abs() + 0.5           # positive, so row 5's sum is +inf
     x[3, 100] = 0.0             # ... except column 100: inf x 0
     w[5, 3] = float("inf")
