@@ -860,7 +860,7 @@ __global__ __launch_bounds__(256) void quant_direct_kernel(const uint8_t* __rest
 // ---------------------------------------------------------------------------
 constexpr int kQ4gA = 8 * 64 * 16;  // A of one 8-block group: [mfma 8][lane 64] x 16 B
 constexpr int kQ4gX = 8 * 8 * 4;    // sub-block sums of x: [block 8][sub-block 8] floats
-constexpr int kQ4gF = 8 * 4;        // 2^(24 - s) per block
+constexpr int kQ4gF = 8 * 4;        // 2^(12 - s) per block
 constexpr int kQ4gBytes = kQ4gA + kQ4gX + kQ4gF;
 constexpr int kQ4MaxGroups = 16;    // K <= 32768 (a workgroup of at most 16 waves)
 
@@ -979,7 +979,9 @@ __global__ __launch_bounds__(1024) void q4k_mfma_kernel(const uint8_t* __restric
     sum += dpp_f32<kDppXor2>(sum);                // the sub-block's 4 chunks
     // am = f 2^e, f in [0.5, 1): am 2^(14 - e) in [2^13, 2^14).  (am = 0, inf,
     // nan: e = 0.)
-    const int s = min(max(14 - __builtin_amdgcn_frexp_expf(am), -100), 140);
+    // 2^(24 - s) goes to the sums in two factors, 2^(12 - s) and 2^12: for x near
+    // the end of the fp32 range it alone would overflow.
+    const int s = min(max(14 - __builtin_amdgcn_frexp_expf(am), -114), 128);
     const float xs[8] = {ldexpf(v0.x, s), ldexpf(v0.z, s), ldexpf(v0.y, s), ldexpf(v0.w, s),
                          ldexpf(v1.x, s), ldexpf(v1.z, s), ldexpf(v1.y, s), ldexpf(v1.w, s)};
     f16x8 hv, mv;
@@ -994,7 +996,7 @@ __global__ __launch_bounds__(1024) void q4k_mfma_kernel(const uint8_t* __restric
     *(f16x8*)(gb + (mf * 64 + 16 * ct + 2 * bb) * 16) = hv;
     *(f16x8*)(gb + (mf * 64 + 16 * ct + 2 * bb + 1) * 16) = mv;
     if ((cb & 3) == 0) ((float*)(gb + kQ4gA))[bb * 8 + (cb >> 2)] = sum;  // sub-block 2t + h
-    if (cb == 0) ((float*)(gb + kQ4gA + kQ4gX))[bb] = ldexpf(1.0f, 24 - s);
+    if (cb == 0) ((float*)(gb + kQ4gA + kQ4gX))[bb] = ldexpf(1.0f, 12 - s);
   };
   // All of this thread's x chunks (at most 4: a workgroup has at least one
   // wave per group; NORM: one, with its res and nrm chunks), then the first
@@ -1078,7 +1080,7 @@ __global__ __launch_bounds__(1024) void q4k_mfma_kernel(const uint8_t* __restric
       }
       const float vh = odd ? c[2] : c[0], vm = odd ? c[3] : c[1];
       float a = -dmin * fmaf(mn0, X.x, mn1 * X.y);
-      if (diag) a = fmaf(d * fblk, fmaf(vm, 0x1p-11f, vh), a);
+      if (diag) a = fmaf(d * 4096.f, fmaf(vm, 0x1p-11f, vh) * fblk, a);
       a = half_row_sum(a);  // lanes n < 8: row 0 of the pair, n >= 8: row 1
       const int pm = PAIR ? (k & 1) : 0, q = st + (PAIR ? k >> 1 : k) * nstream;
       if ((lane & 7) == 0 && lane < 16 && 2 * q + rr < nrows)

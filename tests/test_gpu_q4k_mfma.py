@@ -59,7 +59,7 @@ def scaled_x(orc, K, seed, mags):
 
 
 @pytest.mark.parametrize("M", [8192, 8193])
-@pytest.mark.parametrize("kind", ["spread", "huge_tiny", "zeros", "subnormal", "mixed_in_block"])
+@pytest.mark.parametrize("kind", ["spread", "huge_tiny", "zeros", "subnormal", "mixed_in_block", "largest"])
 def test_q4k_mfma_x_range(hl, orc, launches, kind, M):
     """Per-block scaling: each block's largest |x| maps to [2^13, 2^14), so
     blocks of any magnitude keep 22 significant bits (8193 rows; 8192 run the
@@ -77,12 +77,14 @@ def test_q4k_mfma_x_range(hl, orc, launches, kind, M):
         x[::7] = 0.0
     elif kind == "subnormal":   # fp32 subnormals only
         x = scaled_x(orc, K, 8204, [1e-40])
+    elif kind == "largest":     # near the end of the fp32 range, beside 1
+        x = scaled_x(orc, K, 8206, [5e34, 1.0])
     else:                       # 1e4 and 1e-4 in one block
         x = orc.normal(K, 8205)
         x[::2] *= 1e4
         x[1::2] *= 1e-4
     got, ref = run(orc, raw, x, M, K)
-    if kind in ("spread", "huge_tiny"):
+    if kind in ("spread", "huge_tiny", "largest"):
         # every block's own part, not only the largest one, is checked: the
         # rows' sums restricted to each magnitude class
         W = orc.dequant_rows(12, raw, M, K).astype(np.float64)
