@@ -623,18 +623,18 @@ inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // The split GEMM's variants: tile, workgroups resident on a CU, and the model
 // of their time by which one is chosen, in us:
 //   2 + rounds of workgroups * (fixed + K / 1000 * (only round ? one : more)).
-// On 80 timed shapes (256 .. 14336 rows and k, 2 .. 4096 columns) the choice is
-// 0.7% off the best of the four on average, 20% at worst; always taking one
-// would cost 1.35 to 1.85 times as much on average.
+// Fitted to 200 timed shapes (4 .. 14336 rows, 2 .. 14336 k, 2 .. 4096 columns):
+// the choice is 0.2% off the best of the four on average, 7% at worst; always
+// taking one would cost 1.35 to 1.9 times as much on average.
 struct SplitVariant {
   int bm, bn, per_cu;
   float fixed, one, more;
 };
 constexpr SplitVariant kSplit[] = {
-    {32, 32, 1, 1.39f, 3.91f, 5.15f},    // 8 waves
-    {64, 64, 1, 3.51f, 7.56f, 9.86f},    // 8 waves
-    {64, 64, 2, 4.46f, 13.33f, 11.67f},  // 4 waves
-    {64, 128, 1, 5.57f, 11.78f, 11.37f}, // 4 waves
+    {32, 32, 1, 2.57f, 4.58f, 4.90f},    // 8 waves
+    {64, 64, 1, 3.80f, 10.39f, 13.15f},  // 8 waves
+    {64, 64, 2, 3.61f, 15.37f, 15.70f},  // 4 waves
+    {64, 128, 1, 8.80f, 14.06f, 12.22f}, // 4 waves
 };
 
 LinearPlan linear_plan(const LinearCall& c) {
@@ -652,7 +652,8 @@ LinearPlan linear_plan(const LinearCall& c) {
     const long long all = tm[0] + tm[1] + tm[2], tn = ((long long)c.T + s.bn - 1) / s.bn;
     if (all * tn > 0x7FFFFFFFLL) continue;
     const long long rounds = (all * tn + (long long)cus * s.per_cu - 1) / ((long long)cus * s.per_cu);
-    const float t = 2.f + (float)rounds * (s.fixed + (rounds > 1 ? s.more : s.one) * (float)c.K * 1e-3f);
+    float t = 2.f + (float)rounds * (s.fixed + (rounds > 1 ? s.more : s.one) * (float)c.K * 1e-3f);
+    if (c.pair && s.bn == 128) t *= 1.1f;  // gate and up of 8192 x 2048, 301 columns: 159 us, on 64x64 tiles 155
     if (p.tiles_m == 0 || t < best) {
       best = t;
       p.variant = v;

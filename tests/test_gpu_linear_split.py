@@ -55,7 +55,7 @@ SHAPES = [(*s, kind) for kind, shapes in {
     _lib.HL_LK_SPLIT_64X64_W8: [(2048, 512, 301), (2081, 545, 257), (2111, 97, 303)],
     _lib.HL_LK_SPLIT_64X64_W4: [(8192, 256, 301), (8225, 129, 333), (4096, 256, 1000), (4133, 161, 1027),
                                 (3001, 191, 2049)],
-    _lib.HL_LK_SPLIT_64X128: [(2048, 1024, 1000), (2033, 1003, 1021), (2001, 1031, 1024), (1985, 1489, 1009)],
+    _lib.HL_LK_SPLIT_64X128: [(4096, 1600, 1000), (4033, 1603, 1021), (3969, 1611, 1024), (3905, 2001, 901)],
 }.items() for s in shapes]
 
 
@@ -68,7 +68,7 @@ def test_edges(hl, launches, M, K, T, kind):
 
 
 # One shape for each tile (two for the 64 x 64 one of four waves).
-TILES = [(96, 700, 45), (2048, 600, 301), (8225, 270, 333), (4096, 300, 1000), (2033, 1003, 1021)]
+TILES = [(96, 700, 45), (2048, 600, 301), (8225, 270, 333), (4096, 300, 1000), (4033, 1603, 1021)]
 
 
 @pytest.mark.parametrize("M,K,T", TILES)
