@@ -16,7 +16,6 @@
 // size is not a multiple of 4 (Q8_0 with K % 64, Q6_K with K % 512) load
 // bytes instead of dwords.
 #include <algorithm>
-#include <climits>
 
 #include "common.h"
 #include "launch.h"
@@ -1118,9 +1117,9 @@ __global__ __launch_bounds__(1024) void q4k_mfma_kernel(const uint8_t* __restric
   }
 }
 
-// What the int8 kernel does not take: K < 2048 or > 4096, fewer weights than
-// i8_from, rows not on 16 bytes, and row counts that leave its last round of
-// workgroups mostly empty.  The MFMA kernel pays for its x prologue (~2 us of latency before the
+// What the int8 kernel does not take: K < 2048 or > 16384, rows not on 16
+// bytes, and row counts that leave its last round of workgroups mostly empty
+// (8193 x 4096; pairs of 8195 x 2048).  The MFMA kernel pays for its x prologue (~2 us of latency before the
 // first product) on matrices of 2^25 weights and more: 14336 x 4096 10.8 us
 // against 15.7, 4096 x 14336 14.2 against 17.0, but 4096 x 4096 8.3 against
 // 6.6 (kernel durations).  A fused pair streams both matrices behind one x
@@ -1188,8 +1187,8 @@ void launch_direct(const uint8_t* w, const float* x, float* y, int M, int K, hip
 // The int8 matrix-core kernel (linear_quant_i8.hip) has 1.3-3 us more of
 // fixed cost than the direct kernel (x to digits, LDS stages) and streams
 // 4.2-6.3 TB/s where that reaches 2.2-3.6 (its VALU work per weight): it
-// takes over from 2^25 weights on (i8_from), a pair counting both matrices.
-// us, direct -> int8:
+// takes over at 2^25 weights, a pair counting both matrices.  us, direct (or
+// q4k_mfma_kernel for Q4_K) -> int8:
 //                     Q4_K          Q5_K          Q6_K          Q8_0
 //   4096 x 4096       5.4 ->  6.6   5.8 ->  7.1   7.5 ->  8.5   7.3 ->  8.2
 //   2x 4096 x 4096    8.4 ->  8.3  10.2 ->  9.2  11.3 -> 11.5  12.1 -> 10.5
@@ -1200,26 +1199,7 @@ void launch_direct(const uint8_t* w, const float* x, float* y, int M, int K, hip
 // With the residual and RMSNorm folded in (two launches before, q4k_mfma's
 // own fold from 2^25), from 2^22 weights on: 2x 2048 x 2048 Q4_K 6.6 -> 5.5,
 // 2x 8192 x 2048 9.0 -> 8.5, 2x 14336 x 4096 16.8 -> 15.2.
-constexpr long long kI8NormWeights = 1LL << 22;
-
-// Weights from which the int8 kernel is the faster one.
-//   Q4_K, q4k_mfma_kernel -> int8.  K = 2048: 49100 rows 12.7 -> 13.9 us, 65500
-//   15.8 -> 15.9, 81900 18.9 -> 18.3.  K <= 3328: 15836 x 2304 13% faster, 14009 x 2560
-//   4%.  K = 3840 and 4096: 12280 x 4096 8.5 -> 9.7, 2x 7974 x 3840 10.1 -> 10.9,
-//   16380 x 4096 11.6 -> 10.7.  Wider, in several steps a row: 3.5% slower on
-//   average (34 shapes, 0.85x to 1.07x), never taken.
-//   Q6_K pays later (2x 4096 x 4096: 11.3 us either way), Q8_0 only from K =
-//   4096 or 1.5 2^25 on (2x 6400 x 2816: 13.9 against 14.9).
-template <int QT>
-long long i8_from(int K) {
-  constexpr long long w = 1LL << 25;
-  switch (QT) {
-    case HL_GGML_Q4_K: return K <= 2048 ? 4 * w : K < 3584 ? w : K <= 4096 ? 2 * w : LLONG_MAX;
-    case HL_GGML_Q6_K: return 40000000;
-    case HL_GGML_Q8_0: return K < 4096 ? 3 * w / 2 : w;
-    default: return w;
-  }
-}
+constexpr long long kI8Weights = 1LL << 25, kI8NormWeights = 1LL << 22;
 
 template <int QT>
 bool try_i8(bool pair, int nmat, const uint8_t* const* w, float* const* y, const int* rows, const float* x, int K,
@@ -1233,7 +1213,11 @@ bool try_i8(bool pair, int nmat, const uint8_t* const* w, float* const* y, const
       c.y[i] = y[i];
       c.rows[i] = rows[i];
     }
-    if (total < i8_from<QT>(K)) return false;
+    // Q6_K pays later (2x 4096 x 4096: 11.3 us either way), Q8_0 only from K =
+    // 4096 or 1.5 2^25 on (2x 6400 x 2816: 13.9 against 14.9).
+    if (total < kI8Weights || (QT == HL_GGML_Q6_K && total < 40000000) ||
+        (QT == HL_GGML_Q8_0 && K < 4096 && total < kI8Weights * 3 / 2))
+      return false;
     c.qtype = QT;
     c.K = K;
     c.nmat = nmat;

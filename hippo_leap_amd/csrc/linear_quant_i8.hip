@@ -487,8 +487,7 @@ bool launch(QmArgs a, int nsb, hipStream_t stream) {
 template <int QT, int MAX, int XQ>
 bool launch_forms(const QmArgs& a, bool pair, int nsb, hipStream_t stream) {
   if (a.res) return pair ? launch<QT, MAX, true, true, XQ>(a, nsb, stream) : launch<QT, MAX, false, true, XQ>(a, nsb, stream);
-  if constexpr (QT == HL_GGML_Q4_K && XQ > 1) return false;  // q4k_mfma_kernel's
-  else return pair ? launch<QT, MAX, true, false, XQ>(a, nsb, stream) : launch<QT, MAX, false, false, XQ>(a, nsb, stream);
+  return pair ? launch<QT, MAX, true, false, XQ>(a, nsb, stream) : launch<QT, MAX, false, false, XQ>(a, nsb, stream);
 }
 
 // K goes to steps of 16 superblocks and a rest, or to as many equal steps

@@ -1,6 +1,7 @@
 """GPU parity of the Q4_K GEMV on the fp16 matrix cores (matrices of 2^25 weights
-and more that the int8 kernel does not take, wide ones above all:
-hl_gpu_linear_col_quant and the fused gate/up and K/V pairs,
+and more that the int8 kernel leaves to it, wide ones and those whose rows would
+leave that one's last round mostly empty; a few cases beside them now run the
+int8 kernel: hl_gpu_linear_col_quant and the fused gate/up and K/V pairs,
 backends/naive.nim:1580-1592, 1905-1920, 1799-1814) against the oracle's
 dequantised rows (quant.nim dequantRowQ4K :244-277) and an fp64 product.
 
@@ -20,7 +21,7 @@ from util import TOL_F32, rel_err
 pytestmark = pytest.mark.gpu
 
 SHAPES = [
-    (8192, 4096),    # exactly 2^25 weights
+    (8192, 4096),    # exactly 2^25 weights (the int8 kernel)
     (8193, 4096),    # odd M: the last row pair has one row
     (6554, 5120),    # 20 blocks: a group of 4 blocks after two of 8
     (2731, 12288),   # six groups
@@ -46,7 +47,7 @@ def test_q4k_mfma_shapes(hl, orc, launches, shape):
     raw = random_rows(rng, 12, M, K)
     got, ref = run(orc, raw, orc.normal(K, 8100 + M), M, K)
     assert rel_err(got, ref) < TOL_F32
-    assert launches(_lib.HL_LK_QUANT if M == 1025 else _lib.HL_LK_Q4K_MFMA) == 1
+    assert launches({8192: _lib.HL_LK_I8, 1025: _lib.HL_LK_QUANT}.get(M, _lib.HL_LK_Q4K_MFMA)) == 1
 
 
 def scaled_x(orc, K, seed, mags):
@@ -57,11 +58,13 @@ def scaled_x(orc, K, seed, mags):
     return x.astype(np.float32)
 
 
+@pytest.mark.parametrize("M", [8192, 8193])
 @pytest.mark.parametrize("kind", ["spread", "huge_tiny", "zeros", "subnormal", "mixed_in_block", "largest"])
-def test_q4k_mfma_x_range(hl, orc, launches, kind):
+def test_q4k_mfma_x_range(hl, orc, launches, kind, M):
     """Per-block scaling: each block's largest |x| maps to [2^13, 2^14), so
-    blocks of any magnitude keep 22 significant bits."""
-    M, K = 8192, 4096
+    blocks of any magnitude keep 22 significant bits (8193 rows; 8192 run the
+    int8 kernel)."""
+    K = 4096
     print(f"q4k mfma x range: {kind}", flush=True)
     rng = np.random.default_rng(8200)
     raw = random_rows(rng, 12, M, K)
@@ -92,10 +95,10 @@ def test_q4k_mfma_x_range(hl, orc, launches, kind):
             g2, r2 = run(orc, raw, xs, M, K)
             assert rel_err(g2, r2) < TOL_F32, f"class 1e{cls:.0f}"
     assert rel_err(got, ref) < TOL_F32
-    assert launches(_lib.HL_LK_Q4K_MFMA) > 0 == launches(_lib.HL_LK_I8)
+    assert launches(_lib.HL_LK_I8 if M == 8192 else _lib.HL_LK_Q4K_MFMA) > 0 == launches(_lib.HL_LK_QUANT)
 
 
-@pytest.mark.parametrize("M", [8192, 16391])  # fp16 kernel, int8 kernel
+@pytest.mark.parametrize("M", [8192, 8193])  # int8 kernel, fp16 kernel
 def test_q4k_mfma_graph_replay(hl, orc, launches, M):
     """Captured in a HIP graph and replayed with new x in between: every
     replay matches an eager call on the same inputs."""
@@ -125,7 +128,7 @@ def test_q4k_mfma_graph_replay(hl, orc, launches, M):
         A.gpu_linear_col_quant(ref, x, w, K, M, 12)
         torch.cuda.synchronize()
         assert torch.equal(y, ref), f"replay {i}"
-    assert launches(_lib.HL_LK_Q4K_MFMA if M == 8192 else _lib.HL_LK_I8) == 6
+    assert launches(_lib.HL_LK_I8 if M == 8192 else _lib.HL_LK_Q4K_MFMA) == 6
 
 
 @pytest.mark.parametrize("M,K", [(8192, 4096), (8195, 4096), (8193, 2048), (8195, 2048)])

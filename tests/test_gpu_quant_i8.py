@@ -1,5 +1,5 @@
-"""GPU: the int8 matrix-core GEMV (Q4_K, Q5_K, Q6_K, Q8_0 matrices from 2^25
-weights on through hl_gpu_linear_col_quant, the fused gate/up and K/V
+"""GPU: the int8 matrix-core GEMV (Q4_K, Q5_K, Q6_K, Q8_0 matrices of 2^25
+weights and more through hl_gpu_linear_col_quant, the fused gate/up and K/V
 entry points) against the oracle's dequantisers and float64 products, at row
 counts off the 16-row groups and widths of one and several steps.
 
@@ -47,29 +47,18 @@ def _close(got, ref):
 
 SHAPES = [(20471, 2048), (20200, 2304), (16375, 3840), (12279, 4096), (12200, 4352), (8187, 4864), (4087, 8704),
           (4081, 14336), (4090, 16384)]
-# What the int8 kernel does not pay for (or take: Q6_K of other than multiples
-# of eight superblocks) runs on the vector ALUs, of Q4_K on the fp16 matrix
-# cores; shapes that it takes are added where these are left out.
-SHAPES_OF = {Q4_K: SHAPES + [(71519, 2048), (12279, 2816), (20471, 3328), (20473, 3840), (16391, 4096)],
-             Q5_K: SHAPES,
-             Q6_K: SHAPES + [(8180, 6144), (8187, 8192), (7999, 10240)],
+# Q6_K takes multiples of eight superblocks and 40 million weights, Q8_0 below
+# K = 4096 1.5 2^25 weights; the others of these run on the vector ALUs.
+SHAPES_OF = {Q4_K: SHAPES, Q5_K: SHAPES,
+             Q6_K: SHAPES + [(8180, 6144), (8187, 8192)],
              Q8_0: SHAPES + [(24583, 2048), (23000, 2304), (27999, 2304)]}
-PAIRS = [(12283, 2048), (6139, 4096), (6100, 4352), (4093, 8192), (4083, 14336)]
-PAIRS_OF = {Q4_K: PAIRS + [(40955, 2048), (8739, 2304), (10239, 3328), (8739, 3840), (8197, 4096)],
-            Q5_K: PAIRS,
-            Q6_K: PAIRS + [(8190, 6144)],
-            Q8_0: PAIRS + [(12300, 2048), (14331, 2304)]}
-LEFT_OUT = {Q4_K: [s for s in SHAPES + PAIRS if s != (20200, 2304)],
-            Q5_K: [],
-            Q6_K: [s for s in SHAPES + PAIRS if s[1] in (2304, 3840, 4352, 4864, 8704)],
-            Q8_0: [(20471, 2048), (20200, 2304), (12283, 2048)]}
+ON_ALUS = [(Q6_K, M, K) for M, K in SHAPES if K in (2304, 3840, 4352, 4864, 8704)] + [
+    (Q8_0, 20471, 2048), (Q8_0, 20200, 2304), (Q8_0, 12283, 2048), (Q6_K, 6100, 4352)]
 
 
 def _took(launches, qtype, M, K, n):
-    kind = _lib.HL_LK_I8
-    if (M, K) in LEFT_OUT[qtype]:
-        kind = _lib.HL_LK_Q4K_MFMA if qtype == Q4_K else _lib.HL_LK_QUANT
-    assert launches(kind) == n
+    alus = (qtype, M, K) in ON_ALUS
+    assert (launches(_lib.HL_LK_QUANT), launches(_lib.HL_LK_I8)) == ((n, 0) if alus else (0, n))
 
 
 @pytest.mark.parametrize("qtype,M,K", [(q, *s) for q, shapes in SHAPES_OF.items() for s in shapes])
@@ -86,6 +75,10 @@ def test_one(hl, orc, launches, qtype, M, K):
     A.gpu_linear_col_quant(again, x, w, K, M, qtype)
     assert torch.equal(again, y[:M])
     _took(launches, qtype, M, K, 2)
+
+
+PAIRS = [(12283, 2048), (6139, 4096), (6100, 4352), (4093, 8192), (4083, 14336)]
+PAIRS_OF = {Q4_K: PAIRS, Q5_K: PAIRS, Q6_K: PAIRS + [(8190, 6144)], Q8_0: PAIRS + [(12300, 2048), (14331, 2304)]}
 
 
 @pytest.mark.parametrize("qtype,M,K", [(q, *s) for q, shapes in PAIRS_OF.items() for s in shapes])
@@ -110,8 +103,7 @@ def test_pairs(hl, orc, launches, qtype, M, K):
     _took(launches, qtype, M, K, 2)
 
 
-@pytest.mark.parametrize("qtype,M", [(Q4_K, 20480), (Q4_K, 71519), (Q5_K, 20480), (Q6_K, 20480),
-                                      (Q8_0, 20480), (Q8_0, 24583)])
+@pytest.mark.parametrize("qtype,M", [(Q4_K, 20480), (Q5_K, 20480), (Q6_K, 20480), (Q8_0, 20480), (Q8_0, 24583)])
 def test_large_and_non_finite_x(hl, orc, launches, qtype, M):
     """x up to the fp32 range is held to 2^-31 of its superblock's largest; an
     inf or NaN in x makes every row NaN (q x summed with its offset or min, as
@@ -127,5 +119,5 @@ def test_large_and_non_finite_x(hl, orc, launches, qtype, M):
         x[700] = bad
         A.gpu_linear_col_quant(y, x, w, K, M, qtype)
         assert bool(torch.isnan(y).all())
-    kind = {(Q4_K, 20480): _lib.HL_LK_Q4K_MFMA, (Q8_0, 20480): _lib.HL_LK_QUANT}.get((qtype, M), _lib.HL_LK_I8)
-    assert launches(kind) == 3
+    alus = (qtype, M) == (Q8_0, 20480)
+    assert launches(_lib.HL_LK_QUANT if alus else _lib.HL_LK_I8) == 3
