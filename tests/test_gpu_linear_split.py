@@ -133,6 +133,21 @@ def test_small_parts(hl, M, K, T):
     _check(w, x, fp32=True)
 
 
+@pytest.mark.parametrize("M,K,T", TILES)
+def test_lost_bits(hl, M, K, T):
+    """Elements with bits below the parts' range among ordinary ones, and one
+    that a partner of 2^100 brings up."""
+    print(f"split gemm lost bits M={M} K={K} T={T}", flush=True)
+    w, x = _operands(M, K, T, 11)
+    x[::3, ::2] *= 2.0 ** -125
+    w[1::5, ::7] = 2.0 ** -140
+    _check(w, x, fp32=True)
+    x[:, 5] = 0.0
+    x[7, 5] = 2.0 ** -120 * (1.0 + 2.0 ** -20)
+    w[:, 7] = 2.0 ** 100
+    _check(w, x, fp32=True)
+
+
 def test_longest_rows(hl):
     """Rows so long that an element's offset inside a tile needs more than 32
     bits (138.6 million columns: row 31 starts behind 2^32)."""
